@@ -18,7 +18,7 @@ import torch
 # host-sanitized one that tests/test_host_sanitizers.py runs the ABI checks on).
 LIB_PATH = pathlib.Path(os.environ.get("CAB_HIP_LIB") or
                         pathlib.Path(__file__).resolve().with_name("libcab_hip.so"))
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 CAB_OK, CAB_EINVAL, CAB_EDTYPE, CAB_ESHAPE, CAB_EWORKSPACE, CAB_EHIP = range(6)
 CAB_F32, CAB_F16, CAB_BF16 = 0, 1, 2
@@ -66,6 +66,13 @@ SIGNATURES = {
     "cab_attn_key_scores": (ctypes.c_int, [_ptr, _ptr, _ptr, ctypes.c_int, _i64, _i64, _i64, _i64,
                                            _i64, _i64, _i64x4, _i64x4, _f32, ctypes.c_int, _ptr,
                                            _i64x4, ctypes.c_int, _ptr]),
+    "cab_flash_attn_scores_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int, _i64, _i64, _i64, _i64,
+                                                                _i64, _i64, _i64x4, _i64x4,
+                                                                ctypes.c_int]),
+    "cab_flash_attn_scores_fwd": (ctypes.c_int, [_ptr, _ptr, _ptr, ctypes.c_int, _i64, _i64, _i64,
+                                                 _i64, _i64, _i64, _i64x4, _i64x4, _i64x4, _i64x4,
+                                                 _f32, ctypes.c_int, _ptr, _ptr, _ptr, _i64x4, _i64,
+                                                 _ptr, _i64x4, _ptr, ctypes.c_size_t, _ptr]),
     "cab_evict_select_workspace_bytes": (ctypes.c_size_t, [_i64]),
     "cab_evict_select": (ctypes.c_int, [_ptr, _i64, _ptr, _i64, _i32, _i32, _i32, ctypes.c_int,
                                         ctypes.c_int, _ptr, _ptr, _ptr, _ptr, ctypes.c_size_t,

@@ -4,10 +4,10 @@ Same module path, names and call contract as the reference's
 ``cab_attention/kernels/flash_attention_accumulate.py``:
 ``flash_attention_with_cumulative_scores`` (:172-261),
 ``FlashAttentionWithAccumulation`` (:264-363), ``get_all_cumulative_scores``
-(:548-598) and ``repeat_kv`` (:470-481). The work runs in two HIP calls:
-``cab_flash_attn_fwd`` (attention output and each query's log-sum-exp) and
-``cab_attn_key_scores`` (each key's total softmax probability over the
-queries).
+(:548-598) and ``repeat_kv`` (:470-481). The work runs in one HIP call,
+``cab_flash_attn_scores_fwd`` (attention output, each query's log-sum-exp and
+each key's total softmax probability over the queries, added to the running
+totals); ``cab_attn_key_scores`` computes the totals alone from a saved lse.
 
 Two deliberate differences from the reference kernel (:23-169):
 
@@ -37,7 +37,7 @@ from .. import _native as nat
 def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float | None = None,
                     causal: bool = False, out: torch.Tensor | None = None,
                     return_lse: bool = False):
-    """Dense attention ``softmax(q k^T * scale) v`` (``cab_flash_attn_fwd``).
+    """Dense attention ``softmax(q k^T * scale) v`` (``cab_flash_attn_scores_fwd``).
 
     q: ``[B, H, N_q, D]``; k, v: ``[B, H_kv, N_k, D]`` with ``H % H_kv == 0``
     (query head h reads K / V head ``h // (H // H_kv)``); D = 64 or 128; bf16, fp16
@@ -45,17 +45,33 @@ def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: fl
     the output ``[B, H, N_q, D]`` and, with ``return_lse``, the fp32
     natural-log log-sum-exp ``[B, H, N_q]``.
     """
+    if out is not None and (tuple(out.shape) != tuple(q.shape) or out.dtype != q.dtype):
+        _check_dense(q, k, v)
+        raise ValueError("out must match q's shape and dtype")
+    out, lse = _dense(q, k, v, scale, causal, out=out, want_lse=return_lse)
+    return (out, lse) if return_lse else out
+
+
+def _check_dense(q, k, v):
     if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
         raise ValueError("q, k, v must be [B, H, N, D]")
     if k.shape != v.shape:
         raise ValueError(f"k and v shapes differ: {tuple(k.shape)} vs {tuple(v.shape)}")
-    B, H, N_q, D = q.shape
+    B, _, _, D = q.shape
     if k.shape[0] != B or k.shape[3] != D:
         raise ValueError(f"k / v must be [B={B}, H_kv, N_k, D={D}]; got {tuple(k.shape)}")
     if not (q.dtype == k.dtype == v.dtype):
         raise TypeError("q, k, v dtypes differ")
+
+
+def _dense(q, k, v, scale, causal, out=None, want_lse=False, old=None, scores=None):
+    """One ``cab_flash_attn_scores_fwd`` call: (out, lse or None), and with
+    ``scores`` (fp32 ``[B, H, N_k]``) the totals, added to ``old`` (fp32
+    ``[B, H, n <= N_k]`` or None)."""
+    _check_dense(q, k, v)
+    B, H, N_q, D = q.shape
     H_kv, N_k = k.shape[1], k.shape[2]
-    dev = nat.require_device(q, k, v)
+    dev = nat.require_device(q, k, v, *(t for t in (old, scores) if t is not None))
     lib = nat.load()
     dt = nat.dtype_code(q)
     q = nat.aligned_rows(q)
@@ -63,21 +79,23 @@ def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: fl
     v = nat.aligned_rows(v)
     if out is None:
         out = torch.empty((B, H, N_q, D), dtype=q.dtype, device=dev)
-    elif tuple(out.shape) != (B, H, N_q, D) or out.dtype != q.dtype:
-        raise ValueError("out must match q's shape and dtype")
-    lse = torch.empty((B, H, N_q), dtype=torch.float32, device=dev) if return_lse else None
+    lse = torch.empty((B, H, N_q), dtype=torch.float32, device=dev) if want_lse else None
     if scale is None:
         scale = 1.0 / math.sqrt(D)
-    wbytes = lib.cab_flash_attn_workspace_bytes(dt, B, H_kv, N_k, D)
+    ks, vs = nat.strides4(k), nat.strides4(v)
+    wbytes = lib.cab_flash_attn_scores_workspace_bytes(dt, B, H, H_kv, N_q, N_k, D, ks, vs,
+                                                       int(scores is not None))
     ws = torch.empty(max(int(wbytes), 16), dtype=torch.uint8, device=dev)
     with torch.cuda.device(dev):
-        st = lib.cab_flash_attn_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), dt, B, H, H_kv, N_q,
-                                    N_k, D, nat.strides4(q), nat.strides4(k), nat.strides4(v),
-                                    nat.strides4(out), float(scale), int(bool(causal)),
-                                    out.data_ptr(), nat.ptr(lse), ws.data_ptr(), ws.numel(),
-                                    nat.stream_ptr(dev))
-    nat.check("cab_flash_attn_fwd", st)
-    return (out, lse) if return_lse else out
+        st = lib.cab_flash_attn_scores_fwd(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), dt, B, H, H_kv, N_q, N_k, D,
+            nat.strides4(q), ks, vs, nat.strides4(out), float(scale), int(bool(causal)),
+            out.data_ptr(), nat.ptr(lse), nat.ptr(old), None if old is None else nat.strides4(old),
+            0 if old is None else old.shape[2], nat.ptr(scores),
+            None if scores is None else nat.strides4(scores), ws.data_ptr(), ws.numel(),
+            nat.stream_ptr(dev))
+    nat.check("cab_flash_attn_scores_fwd", st)
+    return out, lse
 
 
 def key_scores(q: torch.Tensor, k: torch.Tensor, lse: torch.Tensor, scale: float | None = None,
@@ -141,22 +159,23 @@ def flash_attention_with_cumulative_scores(
     """
     B, H, N_q, D = q.shape
     N_k = k.shape[2]
-    out, lse = flash_attention(q, k, v, scale=scale, causal=causal, return_lse=True)
-    if cumulative_scores is None:
-        return out, key_scores(q, k, lse, scale=scale, causal=causal)
+    old = cumulative_scores
+    if old is None:
+        scores = torch.empty((B, H, N_k), dtype=torch.float32, device=q.device)
+        return _dense(q, k, v, scale, causal, scores=scores)[0], scores
     if cumulative_scores.dim() != 3 or tuple(cumulative_scores.shape[:2]) != (B, H):
         raise ValueError(f"cumulative_scores must be [B={B}, H={H}, N]")
-    if cumulative_scores.shape[2] < N_k:
-        extension = torch.zeros(B, H, N_k - cumulative_scores.shape[2], dtype=torch.float32,
-                                device=q.device)
-        cumulative_scores = torch.cat([cumulative_scores.float(), extension], dim=2)
-    elif cumulative_scores.shape[2] > N_k:
-        raise ValueError(f"cumulative_scores has {cumulative_scores.shape[2]} key positions, "
+    if old.shape[2] > N_k:
+        raise ValueError(f"cumulative_scores has {old.shape[2]} key positions, "
                          f"more than N_k={N_k}")
-    if cumulative_scores.dtype != torch.float32 or cumulative_scores.stride(-1) != 1:
-        cumulative_scores = cumulative_scores.float().contiguous()
-    return out, key_scores(q, k, lse, scale=scale, causal=causal, scores=cumulative_scores,
-                           accumulate=True)
+    # Totals as long as the keys are added to where they lie; shorter ones
+    # (new key positions) go to a tensor of the new length.
+    if old.dtype != torch.float32 or old.stride(-1) != 1:
+        old = old.float().contiguous()
+    scores = old
+    if old.shape[2] < N_k:
+        scores = torch.empty((B, H, N_k), dtype=torch.float32, device=q.device)
+    return _dense(q, k, v, scale, causal, old=old, scores=scores)[0], scores
 
 
 class FlashAttentionWithAccumulation(torch.nn.Module):

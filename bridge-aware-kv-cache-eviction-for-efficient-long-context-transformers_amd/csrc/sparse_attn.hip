@@ -48,7 +48,8 @@
 // on a causal diagonal tile). Bound: MFMA.
 #include <cstdlib>
 
-#include "cab_internal.h"
+#include "attn_common.h"
+#include "row_attn.h"
 
 namespace cab {
 namespace {
@@ -114,44 +115,6 @@ struct PackArgs {
   int64_t vs[3];
   int64_t H, N, M;
 };
-
-template <bool BF16>
-__device__ __forceinline__ f32x4 mfma16(const u32x4& a, const u32x4& b, const f32x4& c) {
-  if constexpr (BF16)
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
-                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-}
-
-template <bool BF16>
-__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-  if constexpr (BF16) {
-    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    const bf16x2 v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};  // v_cvt_pk_bf16_f32, RNE
-    return __builtin_bit_cast(uint32_t, v);
-  } else {
-    return static_cast<uint32_t>(f32_to_f16(lo)) | (static_cast<uint32_t>(f32_to_f16(hi)) << 16);
-  }
-}
-
-// fp32 -> bf16 pair split of two values: {hi, lo} with hi = bf16(x) and
-// lo = bf16(x - hi), both round-to-nearest-even (x - hi is exact in fp32).
-__device__ __forceinline__ u32x2 split2(float x0, float x1) {
-  const uint32_t hi = pack2<true>(x0, x1);
-  const float h0 = __builtin_bit_cast(float, hi << 16);
-  const float h1 = __builtin_bit_cast(float, hi & 0xffff0000u);
-  return u32x2{hi, pack2<true>(x0 - h0, x1 - h1)};
-}
-
-// Eight consecutive fp32 values (x0, x1) -> bf16x8 hi and lo operands.
-__device__ __forceinline__ void split8(const f32x4& x0, const f32x4& x1, u32x4& hi, u32x4& lo) {
-  const u32x2 a = split2(x0[0], x0[1]), b = split2(x0[2], x0[3]);
-  const u32x2 e = split2(x1[0], x1[1]), f = split2(x1[2], x1[3]);
-  hi = u32x4{a[0], b[0], e[0], f[0]};
-  lo = u32x4{a[1], b[1], e[1], f[1]};
-}
 
 // One block of V rows in LDS, padded.
 template <int HD>
@@ -270,40 +233,6 @@ __device__ __forceinline__ void dma16(const char* g, char* l) {
   static_assert(OFF >= 0 && OFF < 4096, "global_load_lds immediate offset must be in [0, 4096)");
   __builtin_amdgcn_global_load_lds(g, (lds_void*)l, 16, OFF, 0);
 }
-
-// gfx950 lane swaps between the two halves of two registers (v_permlane32_swap:
-// 32-lane halves; v_permlane16_swap: odd and even 16-lane rows), written as
-// inline asm because the compiler's builtins return the first result twice.
-// The s_nop gives the two wait states a swap needs after a VALU write of
-// its operands.
-__device__ __forceinline__ void lane_swap32(uint32_t& a, uint32_t& b) {
-  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
-}
-__device__ __forceinline__ void lane_swap16(uint32_t& a, uint32_t& b) {
-  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
-}
-
-// Maxima over the four lane groups (lanes c + 16 g, g = 0..3) of two
-// registers at once, without an LDS round trip. In: x0, x1 hold per-lane
-// partial maxima of query column c = lane % 16 for query tiles 0 and 1.
-// Out: each holds its tile's full column maximum in every lane.
-__device__ __forceinline__ void colmax2(float& x0, float& x1) {
-  uint32_t a = __builtin_bit_cast(uint32_t, x0), b = __builtin_bit_cast(uint32_t, x1);
-  lane_swap32(a, b);  // one register holds both tiles' lower halves, the other the upper
-  float y = __builtin_fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
-  // y: tile 0 merged over g and g ^ 2 in one 32-lane half, tile 1 in the other.
-  a = b = __builtin_bit_cast(uint32_t, y);
-  lane_swap16(a, b);  // rows g and g ^ 1 side by side
-  y = __builtin_fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
-  a = b = __builtin_bit_cast(uint32_t, y);
-  lane_swap32(a, b);  // each half broadcast to all 64 lanes
-  x0 = __builtin_bit_cast(float, a);
-  x1 = __builtin_bit_cast(float, b);
-}
-
-// Running-max sentinel: a finite stand-in for -inf, so that -max * c stays
-// finite and exp2(s * c - max * c) of a masked score (-inf) is exactly 0.
-constexpr float M_EMPTY = -1.0e30f;
 
 // Softmax modes of one block step.
 //  SM_ONLINE: online softmax with the lazy rescale (the maximum may grow).
@@ -1442,8 +1371,9 @@ struct KeyScoreArgs {
   const void* k;
   const float* lse;  // [B, H, Nq] contiguous
   float* score;      // score[b * ss0 + h * ss1 + token]
-  int64_t qs[3], ks[3], ss[2];
-  int32_t BH, H, group, Nq, Nk, Mk, Mkg, qoff, causal, accumulate;
+  const float* old;  // added to: old[b * olds0 + h * olds1 + token] for tokens below n_old
+  int64_t qs[3], ks[3], ss[2], olds[2], n_old;
+  int32_t BH, H, group, Nq, Nk, Mk, Mkg, qoff, causal;
   float scale_log2;
 };
 
@@ -1646,8 +1576,8 @@ __global__ __launch_bounds__(64 * NW) void key_score_kernel(KeyScoreArgs a) {
   }
   const int key = j * BS + lane;
   if (has_keys && key < a.Nk) {
-    float* dst = a.score + b * a.ss[0] + hh * a.ss[1] + key;
-    *dst = a.accumulate ? *dst + mine : mine;
+    const float base = key < a.n_old ? a.old[b * a.olds[0] + hh * a.olds[1] + key] : 0.f;
+    a.score[b * a.ss[0] + hh * a.ss[1] + key] = base + mine;
   }
 }
 
@@ -2072,13 +2002,198 @@ cab_status_t check_dense(const char* fn, cab_dtype_t dtype, bool allow_f32, int6
   return CAB_OK;
 }
 
+size_t dense_packed_bytes(cab_dtype_t dtype, int64_t B, int64_t H_kv, int64_t N_k, int64_t D) {
+  return static_cast<size_t>(B * H_kv * ceil_div(N_k, BS)) * block_bytes(dtype, static_cast<int>(D));
+}
+
+// Key totals of one dense call: what they are added to and where they go.
+struct Totals {
+  const float* old = nullptr;  // keys below n_old (may be scores itself), 0 beyond
+  int64_t old_strides[2] = {0, 0}, n_old = 0;
+  float* scores = nullptr;  // null: no totals
+  int64_t strides[2] = {0, 0};
+};
+
+cab_status_t launch_key_scores(const char* fn, const void* q, const void* k, const float* lse,
+                               cab_dtype_t dtype, int64_t B, int64_t H, int64_t H_kv, int64_t N_q,
+                               int64_t N_k, int64_t D, const int64_t* q_strides,
+                               const int64_t* k_strides, float scale, int causal, const Totals& t,
+                               hipStream_t s) {
+  KeyScoreArgs a;
+  a.q = q;
+  a.k = k;
+  a.lse = lse;
+  a.score = t.scores;
+  a.old = t.old;
+  a.n_old = t.old ? t.n_old : 0;
+  for (int d = 0; d < 3; ++d) {
+    a.qs[d] = q_strides[d];
+    a.ks[d] = k_strides[d];
+  }
+  for (int d = 0; d < 2; ++d) {
+    a.ss[d] = t.strides[d];
+    a.olds[d] = t.old_strides[d];
+  }
+  a.BH = static_cast<int32_t>(B * H);
+  a.H = static_cast<int32_t>(H);
+  a.group = static_cast<int32_t>(H / H_kv);
+  a.Nq = static_cast<int32_t>(N_q);
+  a.Nk = static_cast<int32_t>(N_k);
+  a.Mk = static_cast<int32_t>(ceil_div(N_k, BS));
+  a.Mkg = static_cast<int32_t>(ceil_div(a.Mk, KS_WAVES));
+  a.qoff = static_cast<int32_t>(N_k - N_q);
+  a.causal = causal ? 1 : 0;
+  a.scale_log2 = static_cast<float>(static_cast<double>(scale) * 1.4426950408889634);
+  const dim3 grid(static_cast<unsigned>(B * H * a.Mkg));
+  auto launch = [&](auto hd_tag) {
+    constexpr int HDT = decltype(hd_tag)::value;
+    switch (dtype) {
+      case CAB_BF16: key_score_kernel<CAB_BF16, KS_WAVES, HDT><<<grid, 64 * KS_WAVES, 0, s>>>(a); break;
+      case CAB_F16: key_score_kernel<CAB_F16, KS_WAVES, HDT><<<grid, 64 * KS_WAVES, 0, s>>>(a); break;
+      default: key_score_kernel<CAB_F32, KS_WAVES, HDT><<<grid, 64 * KS_WAVES, 0, s>>>(a); break;
+    }
+  };
+  if (D == 64)
+    launch(std::integral_constant<int, 64>{});
+  else
+    launch(std::integral_constant<int, 128>{});
+  return launch_status(fn);
+}
+
+// Checks of the key-total tensors and of what the totals read.
+cab_status_t check_scores(const char* fn, const float* scores, const int64_t* strides) {
+  CAB_REQUIRE(scores != nullptr, CAB_EINVAL, "%s: null scores", fn);
+  CAB_REQUIRE(strides[2] == 1 && strides[0] >= 0 && strides[1] >= 0, CAB_ESHAPE,
+              "%s: scores must have a contiguous token dim", fn);
+  return CAB_OK;
+}
+cab_status_t check_score_rows(const char* fn, const void* q, const float* lse,
+                              const int64_t* q_strides, int64_t esize) {
+  cab_status_t st;
+  if ((st = check_tensor(fn, "q", q, q_strides, esize)) != CAB_OK) return st;
+  CAB_REQUIRE(lse != nullptr && reinterpret_cast<uintptr_t>(lse) % 4 == 0, CAB_EINVAL,
+              "%s: lse must be the fp32 [B, H, N_q] rows cab_flash_attn_fwd wrote", fn);
+  // 16 query rows are staged through one buffer descriptor (32-bit offsets).
+  CAB_REQUIRE(q_strides[2] * esize < (int64_t{1} << 27), CAB_ESHAPE,
+              "%s: q token stride of %lld elements exceeds the 2^27-byte limit", fn,
+              (long long)q_strides[2]);
+  return CAB_OK;
+}
+
+// Workspace of the dense path: the few-row kernels' partials, or the packed V
+// (fp32: K and V) and, when the totals need it and the caller keeps no lse,
+// the lse rows.
+struct DensePlan {
+  bool rows;        // the few-row kernels
+  size_t off_lse, bytes;
+};
+DensePlan dense_plan(cab_dtype_t dtype, int64_t B, int64_t H, int64_t H_kv, int64_t N_q,
+                     int64_t N_k, int64_t D, bool rows, bool scores) {
+  DensePlan p;
+  p.rows = rows;
+  p.off_lse = 0;
+  if (rows) {
+    p.bytes = row_attn_workspace(B, H, H_kv, N_q, N_k, D, scores);
+    return p;
+  }
+  p.off_lse = dense_packed_bytes(dtype, B, H_kv, N_k, D);
+  p.bytes = p.off_lse + (scores ? static_cast<size_t>(B * H * N_q) * 4 : 0);
+  return p;
+}
+
+// Dense attention (and the key totals, when t.scores is set) on checked sizes.
+// The few-row kernels run when they take the problem and the workspace holds
+// their partials. least: workspace bytes the entry point asks for in any case.
+cab_status_t dense_forward(const char* fn, const void* q, const void* k, const void* v,
+                           cab_dtype_t dtype, int64_t B, int64_t H, int64_t H_kv, int64_t N_q,
+                           int64_t N_k, int64_t D, const int64_t* q_strides,
+                           const int64_t* k_strides, const int64_t* v_strides,
+                           const int64_t* o_strides, float scale, int causal, void* out,
+                           float* lse, const Totals& t, void* workspace, size_t workspace_bytes,
+                           size_t least, hipStream_t s) {
+  cab_status_t st;
+  const int64_t esize = dtype == CAB_F32 ? 4 : 2;
+  const bool scores = t.scores != nullptr;
+  if ((st = check_tensor(fn, "q", q, q_strides, esize)) != CAB_OK) return st;
+  if ((st = check_tensor(fn, "out", out, o_strides, esize)) != CAB_OK) return st;
+  CAB_REQUIRE(lse == nullptr || reinterpret_cast<uintptr_t>(lse) % 4 == 0, CAB_ESHAPE,
+              "%s: lse not 4-byte aligned", fn);
+  if (N_k == 0 || H_kv == 0) {
+    // No keys: every row attends to nothing (output 0, lse -inf); K, V and
+    // the workspace are not read (q stands in for their addresses).
+    const AttnGeom g{B, H, H_kv > 0 ? H_kv : H, N_q, 0, D, -N_q, LIST_DENSE};
+    return launch_attn(fn, q, q, q, dtype, g, q_strides, q_strides, o_strides, nullptr, nullptr,
+                       1, scale, causal, out, lse, s);
+  }
+  if ((st = check_tensor(fn, "k", k, k_strides, esize)) != CAB_OK) return st;
+  if ((st = check_tensor(fn, "v", v, v_strides, esize)) != CAB_OK) return st;
+  CAB_REQUIRE(k_strides[2] <= (int64_t{1} << 24), CAB_ESHAPE,
+              "%s: k token stride %lld too large (<= 2^24 elements)", fn, (long long)k_strides[2]);
+  CAB_REQUIRE(workspace != nullptr && workspace_bytes >= least, CAB_EWORKSPACE,
+              "%s: workspace of %zu bytes given, %zu needed", fn, workspace_bytes, least);
+  CAB_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16 == 0, CAB_EWORKSPACE,
+              "%s: workspace not 16-byte aligned", fn);
+  if (row_attn_applies(dtype, B, H, H_kv, N_q, N_k, D, k_strides, v_strides) &&
+      workspace_bytes >= dense_plan(dtype, B, H, H_kv, N_q, N_k, D, true, scores).bytes) {
+    RowAttnProblem p{};
+    p.dtype = dtype;
+    p.B = B, p.H = H, p.Hkv = H_kv, p.Nq = N_q, p.Nk = N_k, p.D = D;
+    p.q = q, p.k = k, p.v = v, p.out = out, p.lse = lse;
+    for (int d = 0; d < 3; ++d) {
+      p.qs[d] = q_strides[d];
+      p.ks[d] = k_strides[d];
+      p.vs[d] = v_strides[d];
+      p.os[d] = o_strides[d];
+    }
+    p.scale = scale;
+    p.causal = causal;
+    p.old_scores = t.old;
+    p.n_old = t.n_old;
+    p.scores = t.scores;
+    for (int d = 0; d < 2; ++d) {
+      p.olds[d] = t.old_strides[d];
+      p.ss[d] = t.strides[d];
+    }
+    return row_attn_launch(fn, p, workspace, s);
+  }
+  const DensePlan plan = dense_plan(dtype, B, H, H_kv, N_q, N_k, D, false, scores && !lse);
+  CAB_REQUIRE(workspace_bytes >= plan.bytes, CAB_EWORKSPACE,
+              "%s: workspace of %zu bytes given, %zu needed", fn, workspace_bytes, plan.bytes);
+  if (scores && !lse)
+    lse = reinterpret_cast<float*>(static_cast<char*>(workspace) + plan.off_lse);
+  if (scores && (st = check_score_rows(fn, q, lse, q_strides, esize)) != CAB_OK) return st;
+  if (dtype == CAB_F32)
+    st = launch_pack_split(fn, k, k_strides, v, v_strides, B, H_kv, N_k, D, workspace, s);
+  else
+    st = launch_pack(fn, v, v_strides, B, H_kv, N_k, D, workspace, s);
+  if (st != CAB_OK) return st;
+  const AttnGeom g{B, H, H_kv, N_q, N_k, D, N_k - N_q, LIST_DENSE};
+  st = launch_attn(fn, q, k, workspace, dtype, g, q_strides, k_strides, o_strides, nullptr,
+                   nullptr, 1, scale, causal, out, lse, s);
+  if (st != CAB_OK || !scores) return st;
+  return launch_key_scores(fn, q, k, lse, dtype, B, H, H_kv, N_q, N_k, D, q_strides, k_strides,
+                           scale, causal, t, s);
+}
+
 }  // namespace
 
 extern "C" size_t cab_flash_attn_workspace_bytes(cab_dtype_t dtype, int64_t B, int64_t H_kv,
                                                  int64_t N_k, int64_t D) {
   if (dtype != CAB_BF16 && dtype != CAB_F16 && dtype != CAB_F32) return 0;
   if (B <= 0 || H_kv <= 0 || N_k <= 0 || (D != 64 && D != 128)) return 0;
-  return static_cast<size_t>(B * H_kv * ceil_div(N_k, BS)) * block_bytes(dtype, static_cast<int>(D));
+  return dense_packed_bytes(dtype, B, H_kv, N_k, D);
+}
+
+extern "C" size_t cab_flash_attn_scores_workspace_bytes(cab_dtype_t dtype, int64_t B, int64_t H,
+                                                        int64_t H_kv, int64_t N_q, int64_t N_k,
+                                                        int64_t D, const int64_t k_strides[4],
+                                                        const int64_t v_strides[4], int scores) {
+  if (dtype != CAB_BF16 && dtype != CAB_F16 && dtype != CAB_F32) return 0;
+  if (B <= 0 || H <= 0 || H_kv <= 0 || H % H_kv != 0 || N_q <= 0 || N_k <= 0 ||
+      (D != 64 && D != 128) || !k_strides || !v_strides)
+    return 0;
+  const bool rows = row_attn_applies(dtype, B, H, H_kv, N_q, N_k, D, k_strides, v_strides);
+  return dense_plan(dtype, B, H, H_kv, N_q, N_k, D, rows, scores != 0).bytes;
 }
 
 extern "C" cab_status_t cab_flash_attn_fwd(
@@ -2096,38 +2211,10 @@ extern "C" cab_status_t cab_flash_attn_fwd(
   CAB_REQUIRE(q_strides && k_strides && v_strides && o_strides, CAB_EINVAL,
               "%s: null stride array", fn);
   if (B == 0 || H == 0 || N_q == 0) return CAB_OK;
-  const int64_t esize = dtype == CAB_F32 ? 4 : 2;
-  if ((st = check_tensor(fn, "q", q, q_strides, esize)) != CAB_OK) return st;
-  if ((st = check_tensor(fn, "out", out, o_strides, esize)) != CAB_OK) return st;
-  CAB_REQUIRE(lse == nullptr || reinterpret_cast<uintptr_t>(lse) % 4 == 0, CAB_ESHAPE,
-              "%s: lse not 4-byte aligned", fn);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (N_k == 0 || H_kv == 0) {
-    // No keys: every row attends to nothing (output 0, lse -inf); K, V and
-    // the workspace are not read (q stands in for their addresses).
-    const AttnGeom g{B, H, H_kv > 0 ? H_kv : H, N_q, 0, D, -N_q, LIST_DENSE};
-    return launch_attn(fn, q, q, q, dtype, g, q_strides, q_strides, o_strides, nullptr, nullptr,
-                       1, scale, causal, out, lse, s);
-  }
-  if ((st = check_tensor(fn, "k", k, k_strides, esize)) != CAB_OK) return st;
-  if ((st = check_tensor(fn, "v", v, v_strides, esize)) != CAB_OK) return st;
-  CAB_REQUIRE(k_strides[2] <= (int64_t{1} << 24), CAB_ESHAPE,
-              "%s: k token stride %lld too large (<= 2^24 elements)", fn, (long long)k_strides[2]);
-  const int64_t Mk = ceil_div(N_k, BS);
-  const size_t need = static_cast<size_t>(B * H_kv * Mk) * block_bytes(dtype, static_cast<int>(D));
-  CAB_REQUIRE(workspace != nullptr && workspace_bytes >= need, CAB_EWORKSPACE,
-              "%s: workspace of %zu bytes given, %zu needed", fn, workspace_bytes, need);
-  CAB_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16 == 0, CAB_EWORKSPACE,
-              "%s: workspace not 16-byte aligned", fn);
-  if (dtype == CAB_F32)
-    st = launch_pack_split("cab_flash_attn_fwd/pack_split", k, k_strides, v, v_strides, B, H_kv,
-                           N_k, D, workspace, s);
-  else
-    st = launch_pack("cab_flash_attn_fwd/pack_v", v, v_strides, B, H_kv, N_k, D, workspace, s);
-  if (st != CAB_OK) return st;
-  const AttnGeom g{B, H, H_kv, N_q, N_k, D, N_k - N_q, LIST_DENSE};
-  return launch_attn(fn, q, k, workspace, dtype, g, q_strides, k_strides, o_strides, nullptr,
-                     nullptr, 1, scale, causal, out, lse, s);
+  return dense_forward(fn, q, k, v, dtype, B, H, H_kv, N_q, N_k, D, q_strides, k_strides,
+                       v_strides, o_strides, scale, causal, out, lse, Totals{}, workspace,
+                       workspace_bytes, dense_packed_bytes(dtype, B, H_kv, N_k, D),
+                       static_cast<hipStream_t>(stream));
 }
 
 extern "C" cab_status_t cab_attn_key_scores(
@@ -2144,54 +2231,61 @@ extern "C" cab_status_t cab_attn_key_scores(
   CAB_REQUIRE(q_strides && k_strides && score_strides, CAB_EINVAL, "%s: null stride array", fn);
   const int64_t esize = dtype == CAB_F32 ? 4 : 2;
   if (B == 0 || H == 0 || N_k == 0) return CAB_OK;
-  CAB_REQUIRE(scores != nullptr, CAB_EINVAL, "%s: null scores", fn);
-  CAB_REQUIRE(score_strides[2] == 1 && score_strides[0] >= 0 && score_strides[1] >= 0,
-              CAB_ESHAPE, "%s: scores must have a contiguous token dim", fn);
-  if (N_q > 0) {
-    if ((st = check_tensor(fn, "q", q, q_strides, esize)) != CAB_OK) return st;
-    CAB_REQUIRE(lse != nullptr && reinterpret_cast<uintptr_t>(lse) % 4 == 0, CAB_EINVAL,
-                "%s: lse must be the fp32 [B, H, N_q] rows cab_flash_attn_fwd wrote", fn);
-    // 16 query rows are staged through one buffer descriptor (32-bit offsets).
-    CAB_REQUIRE(q_strides[2] * esize < (int64_t{1} << 27), CAB_ESHAPE,
-                "%s: q token stride of %lld elements exceeds the 2^27-byte limit", fn,
-                (long long)q_strides[2]);
-  }
+  if ((st = check_scores(fn, scores, score_strides)) != CAB_OK) return st;
+  if (N_q > 0 && (st = check_score_rows(fn, q, lse, q_strides, esize)) != CAB_OK) return st;
   if ((st = check_tensor(fn, "k", k, k_strides, esize)) != CAB_OK) return st;
-  KeyScoreArgs a;
-  a.q = q;
-  a.k = k;
-  a.lse = lse;
-  a.score = scores;
-  for (int d = 0; d < 3; ++d) {
-    a.qs[d] = q_strides[d];
-    a.ks[d] = k_strides[d];
+  Totals t;
+  t.scores = scores;
+  t.strides[0] = score_strides[0], t.strides[1] = score_strides[1];
+  if (accumulate) {
+    t.old = scores;
+    t.old_strides[0] = score_strides[0], t.old_strides[1] = score_strides[1];
+    t.n_old = N_k;
   }
-  a.ss[0] = score_strides[0];
-  a.ss[1] = score_strides[1];
-  a.BH = static_cast<int32_t>(B * H);
-  a.H = static_cast<int32_t>(H);
-  a.group = static_cast<int32_t>(H / H_kv);
-  a.Nq = static_cast<int32_t>(N_q);
-  a.Nk = static_cast<int32_t>(N_k);
-  a.Mk = static_cast<int32_t>(ceil_div(N_k, BS));
-  a.Mkg = static_cast<int32_t>(ceil_div(a.Mk, KS_WAVES));
-  a.qoff = static_cast<int32_t>(N_k - N_q);
-  a.causal = causal ? 1 : 0;
-  a.accumulate = accumulate ? 1 : 0;
-  a.scale_log2 = static_cast<float>(static_cast<double>(scale) * 1.4426950408889634);
-  const dim3 grid(static_cast<unsigned>(B * H * a.Mkg));
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  auto launch = [&](auto hd_tag) {
-    constexpr int HDT = decltype(hd_tag)::value;
-    switch (dtype) {
-      case CAB_BF16: key_score_kernel<CAB_BF16, KS_WAVES, HDT><<<grid, 64 * KS_WAVES, 0, s>>>(a); break;
-      case CAB_F16: key_score_kernel<CAB_F16, KS_WAVES, HDT><<<grid, 64 * KS_WAVES, 0, s>>>(a); break;
-      default: key_score_kernel<CAB_F32, KS_WAVES, HDT><<<grid, 64 * KS_WAVES, 0, s>>>(a); break;
+  return launch_key_scores(fn, q, k, lse, dtype, B, H, H_kv, N_q, N_k, D, q_strides, k_strides,
+                           scale, causal, t, static_cast<hipStream_t>(stream));
+}
+
+extern "C" cab_status_t cab_flash_attn_scores_fwd(
+    const void* q, const void* k, const void* v, cab_dtype_t dtype, int64_t B, int64_t H,
+    int64_t H_kv, int64_t N_q, int64_t N_k, int64_t D, const int64_t q_strides[4],
+    const int64_t k_strides[4], const int64_t v_strides[4], const int64_t o_strides[4],
+    float scale, int causal, void* out, float* lse, const float* old_scores,
+    const int64_t old_strides[3], int64_t n_old, float* scores, const int64_t score_strides[3],
+    void* workspace, size_t workspace_bytes, void* stream) {
+  const char* fn = "cab_flash_attn_scores_fwd";
+  clear_error();
+  cab_status_t st = check_dense(fn, dtype, true, B, H, H_kv, N_q, N_k, D);
+  if (st != CAB_OK) return st;
+  CAB_REQUIRE(std::isfinite(scale) && scale > 0.f, CAB_EINVAL, "%s: scale must be finite and > 0",
+              fn);
+  CAB_REQUIRE(q_strides && k_strides && v_strides && o_strides, CAB_EINVAL,
+              "%s: null stride array", fn);
+  if (B == 0 || H == 0) return CAB_OK;
+  Totals t;
+  if (scores != nullptr && N_k > 0) {
+    CAB_REQUIRE(score_strides != nullptr, CAB_EINVAL, "%s: null stride array", fn);
+    if ((st = check_scores(fn, scores, score_strides)) != CAB_OK) return st;
+    t.scores = scores;
+    t.strides[0] = score_strides[0], t.strides[1] = score_strides[1];
+    if (old_scores != nullptr) {
+      CAB_REQUIRE(old_strides != nullptr, CAB_EINVAL, "%s: null stride array", fn);
+      CAB_REQUIRE(n_old >= 0 && n_old <= N_k && old_strides[2] == 1 && old_strides[0] >= 0 &&
+                      old_strides[1] >= 0,
+                  CAB_ESHAPE, "%s: old totals must be [B, H, n_old <= N_k], contiguous in the last "
+                  "dim", fn);
+      t.old = old_scores;
+      t.old_strides[0] = old_strides[0], t.old_strides[1] = old_strides[1];
+      t.n_old = n_old;
     }
-  };
-  if (D == 64)
-    launch(std::integral_constant<int, 64>{});
-  else
-    launch(std::integral_constant<int, 128>{});
-  return launch_status(fn);
+  }
+  if (N_q == 0) {  // no queries: the totals are the old ones
+    if (!t.scores) return CAB_OK;
+    if ((st = check_tensor(fn, "k", k, k_strides, dtype == CAB_F32 ? 4 : 2)) != CAB_OK) return st;
+    return launch_key_scores(fn, q, k, lse, dtype, B, H, H_kv, N_q, N_k, D, q_strides, k_strides,
+                             scale, causal, t, static_cast<hipStream_t>(stream));
+  }
+  return dense_forward(fn, q, k, v, dtype, B, H, H_kv, N_q, N_k, D, q_strides, k_strides,
+                       v_strides, o_strides, scale, causal, out, lse, t, workspace,
+                       workspace_bytes, 0, static_cast<hipStream_t>(stream));
 }

@@ -55,7 +55,7 @@ enum { CAB_NORM_NONE = 0, CAB_NORM_MINMAX = 1 };
 /* FRC combination (experiments/longbench_qa/config.py:465; test.ipynb:111-145). */
 enum { CAB_FRC_ADDITIVE = 0, CAB_FRC_MULTIPLICATIVE = 1, CAB_FRC_AUGMENTED = 2 };
 
-#define CAB_ABI_VERSION 10
+#define CAB_ABI_VERSION 11
 
 int cab_abi_version(void);
 const char* cab_last_error(void);
@@ -291,6 +291,34 @@ cab_status_t cab_attn_key_scores(const void* q, const void* k, const float* lse,
                                  const int64_t k_strides[4], float scale, int causal,
                                  float* scores, const int64_t score_strides[3], int accumulate,
                                  void* stream);
+
+/*
+ * cab_flash_attn_scores_fwd: both of the above in one call, the whole of
+ * flash_attention_with_cumulative_scores (flash_attention_accumulate.py:172-261,
+ * the extension of the running totals to new key positions included):
+ * out and lse (may be NULL) as cab_flash_attn_fwd, and with scores != NULL
+ *   scores[b,h,s] = (s < n_old ? old_scores[b,h,s] : 0) + this call's total.
+ * old_scores: fp32 [B,H,n_old], n_old <= N_k, strides {b, h, 1}, may be NULL
+ * (nothing is added to) and may be scores itself. workspace:
+ * cab_flash_attn_scores_workspace_bytes() bytes for the same sizes and
+ * strides (scores != 0 when totals are asked for), 16-byte aligned,
+ * overwritten. At most 64 rows per K / V head (H / H_kv * N_q; decode steps
+ * and short chunks) run kernels that split the key range over the chip and
+ * read K and V once; so does cab_flash_attn_fwd when its workspace holds
+ * that path's partials.
+ */
+size_t cab_flash_attn_scores_workspace_bytes(cab_dtype_t dtype, int64_t B, int64_t H, int64_t H_kv,
+                                             int64_t N_q, int64_t N_k, int64_t D,
+                                             const int64_t k_strides[4],
+                                             const int64_t v_strides[4], int scores);
+
+cab_status_t cab_flash_attn_scores_fwd(
+    const void* q, const void* k, const void* v, cab_dtype_t dtype, int64_t B, int64_t H,
+    int64_t H_kv, int64_t N_q, int64_t N_k, int64_t D, const int64_t q_strides[4],
+    const int64_t k_strides[4], const int64_t v_strides[4], const int64_t o_strides[4],
+    float scale, int causal, void* out, float* lse, const float* old_scores,
+    const int64_t old_strides[3], int64_t n_old, float* scores, const int64_t score_strides[3],
+    void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * KV-cache eviction: which cache positions to keep, and the pruned cache.
