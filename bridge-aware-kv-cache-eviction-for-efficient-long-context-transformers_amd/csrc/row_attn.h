@@ -28,7 +28,7 @@ struct RowAttnProblem {
 
 // Whether the few-row kernels take this problem's sizes and strides.
 bool row_attn_applies(cab_dtype_t dtype, int64_t B, int64_t H, int64_t Hkv, int64_t Nq, int64_t Nk,
-                      int64_t D, const int64_t* k_strides, const int64_t* v_strides);
+                      int64_t D, const int64_t* k_strides, const int64_t* v_strides, bool scores);
 // Workspace bytes of such a problem (16-byte aligned).
 size_t row_attn_workspace(int64_t B, int64_t H, int64_t Hkv, int64_t Nq, int64_t Nk, int64_t D,
                           bool scores);

@@ -2,7 +2,7 @@
 // of queries against a long key range.
 //
 // The query heads that share a K / V head and their N_q queries are the
-// R = group * N_q rows of one unit (b, K / V head), at most 64. K and V are
+// R = group * N_q rows of one unit (b, K / V head), at most 32. K and V are
 // then read once per unit, straight from their rows, and the key range is
 // split over workgroups so that the chip is full whatever B * H_kv is:
 //  1. row_attn_kernel: grid (split, unit). Each wave walks its own 32-key
@@ -38,7 +38,14 @@ namespace cab {
 namespace {
 
 constexpr int STEP = 32;        // keys per wave step
-constexpr int MAX_ROWS = 64;    // rows per unit
+// Rows per unit, and queries per head when totals are wanted, beyond which the
+// general kernels are as fast or faster (bf16, causal, us, general -> here):
+// 32 rows 28.3 -> 17.5 (32 heads on 8, 8 queries, 4099 keys), 39.0 -> 34.1 (12
+// heads, 8000 keys); 64 rows 28.6 -> 29.4 (32 on 8, 16 queries, 4099 keys). With
+// totals 24 queries 51.6 -> 44.2 (32 heads, 5000 keys), 32 queries 34.0 -> 37.3
+// (32 heads, 2000 keys).
+constexpr int MAX_ROWS = 32;
+constexpr int MAX_TOTAL_QUERIES = 24;
 constexpr int MAX_SPLITS = 256;
 constexpr int KEYS_PER_WG = 1024;  // keys one row_combine workgroup totals
 // Workgroups a plan aims at: two per CU run at a time (512, 1024 and 2048
@@ -128,7 +135,7 @@ struct RowAcc {
 };
 
 template <cab_dtype_t DT, int HD, int QT, bool SC>
-__global__ __launch_bounds__(256, QT * HD > 256 || DT == CAB_F32 ? 1 : 2) void row_attn_kernel(RowArgs a) {
+__global__ __launch_bounds__(256, DT == CAB_F32 ? 1 : 2) void row_attn_kernel(RowArgs a) {
   constexpr bool F32 = DT == CAB_F32;
   constexpr bool BF16 = DT != CAB_F16;
   constexpr int NDS = HD / 32, NDT = HD / 16;
@@ -435,11 +442,12 @@ __global__ __launch_bounds__(256) void row_combine_kernel(CombineArgs a) {
     float sum[PER];
 #pragma unroll
     for (int i = 0; i < PER; ++i) sum[i] = __builtin_amdgcn_exp2f(sv[i] - lse2[0]);
+#pragma unroll 4
     for (int t = 1; t < a.Nq; ++t) {
 #pragma unroll
       for (int i = 0; i < PER; ++i) {
-        const int key = key0 + 256 * i;
-        if (key < a.Nk) sum[i] += __builtin_amdgcn_exp2f(srow[t * a.ld + key] - lse2[t]);
+        const int key = key0 + 256 * i;  // (past the keys: a key of the row, not stored)
+        sum[i] += __builtin_amdgcn_exp2f(srow[t * a.ld + (key < a.Nk ? key : 0)] - lse2[t]);
       }
     }
     float* drow = a.scores + b * a.ss[0] + h * a.ss[1];
@@ -515,17 +523,16 @@ template <cab_dtype_t DT, int HD>
 void launch_dt(const RowArgs& a, dim3 grid, const CombineArgs& ca, dim3 cgrid, hipStream_t s) {
   if (a.R <= 16)
     launch_rows<DT, HD, 1>(a, grid, s);
-  else if (a.R <= 32)
-    launch_rows<DT, HD, 2>(a, grid, s);
   else
-    launch_rows<DT, HD, 4>(a, grid, s);
+    launch_rows<DT, HD, 2>(a, grid, s);
   row_combine_kernel<DT, HD><<<cgrid, 256, 0, s>>>(ca);
 }
 
 }  // namespace
 
 bool row_attn_applies(cab_dtype_t dtype, int64_t B, int64_t H, int64_t Hkv, int64_t Nq, int64_t Nk,
-                      int64_t D, const int64_t* k_strides, const int64_t* v_strides) {
+                      int64_t D, const int64_t* k_strides, const int64_t* v_strides, bool scores) {
+  if (scores && Nq > MAX_TOTAL_QUERIES) return false;
   if (B < 1 || Hkv < 1 || H < Hkv || Nq < 1 || Nk < 1) return false;
   if (H / Hkv * Nq > MAX_ROWS || B * H > 65535) return false;  // grid.y
   // 32 rows of K and of V are addressed by 32-bit offsets.

@@ -107,6 +107,10 @@ struct AttnArgs {
   // k / bs for query q and key k of the tile); null when every tile is whole.
   const uint64_t* submask;
   int sub_shift;  // log2(block_size) when submask is set
+  // LIST_DENSE_SPLIT: splits of each pair's key blocks, and their partials.
+  int32_t splits;
+  float* po;   // [split][BH][N][D] unnormalised O
+  float* pml;  // [2][split][BH][N] running maxima (raw scores), then row sums
 };
 
 struct PackArgs {
@@ -613,7 +617,9 @@ __device__ __forceinline__ uint32_t k_lane_off(int group, int lane, int64_t krow
 // Key-block lists of a query block: the caller's kv_idx staged in LDS, read
 // from global memory (lists longer than LIST_MAX), or dense (every key block
 // up to the causal limit, in order).
-constexpr int LIST_LDS = 0, LIST_GLOBAL = 1, LIST_DENSE = 2;
+// LIST_DENSE_SPLIT (attn_pair_kernel): dense, a workgroup per part of the key
+// blocks, merged by split_combine_kernel.
+constexpr int LIST_LDS = 0, LIST_GLOBAL = 1, LIST_DENSE = 2, LIST_DENSE_SPLIT = 3;
 
 template <cab_dtype_t DT, int LIST, int HD>
 __global__ __launch_bounds__(256, DT == CAB_F32 ? 1 : 2) void attn_fwd_kernel(AttnArgs a) {
@@ -935,8 +941,9 @@ __device__ __forceinline__ void pair_softmax(PairAcc<HD>& s, int r, f32x4 (&sc)[
 template <cab_dtype_t DT, int LIST, int HD>
 __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
   static_assert(DT != CAB_F32, "16-bit inputs only");
-  static_assert(LIST == LIST_LDS || LIST == LIST_DENSE, "lists staged in LDS, or dense");
-  constexpr bool DENSE = LIST == LIST_DENSE;
+  static_assert(LIST != LIST_GLOBAL, "lists staged in LDS, or dense");
+  constexpr bool SPLIT = LIST == LIST_DENSE_SPLIT;
+  constexpr bool DENSE = LIST == LIST_DENSE || SPLIT;
   using G = Dims<HD>;
   constexpr int NDS = G::NDS, NDT = G::NDT;
   constexpr int TILE_SLOTS = G::TILE_SLOTS, TILE_BYTES = G::TILE_BYTES, NI = G::NI;
@@ -954,9 +961,13 @@ __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
 
   const int M = a.M, N = a.N, Mk = a.Mk, Nk = a.Nk;
   const int MP = (M + 1) / 2;
-  const int logical = static_cast<int>(xcd_remap(blockIdx.x, static_cast<int64_t>(a.BH) * MP));
-  const int bh = logical / MP;
-  const int pr = MP - 1 - (logical - bh * MP);  // longest causal pairs first
+  const int logical = static_cast<int>(
+      xcd_remap(blockIdx.x, static_cast<int64_t>(a.BH) * MP * (SPLIT ? a.splits : 1)));
+  // With splits, the pairs of one head and split (the same key blocks) are neighbours.
+  const int bhs = logical / MP;
+  const int bh = SPLIT ? bhs / a.splits : bhs;
+  const int split = SPLIT ? bhs - bh * a.splits : 0;
+  const int pr = MP - 1 - (logical - bhs * MP);  // longest causal pairs first
   const int irow[2] = {2 * pr, 2 * pr + 1};     // irow[1] == M: no second row
   const int b = bh / a.H, hh = bh - (bh / a.H) * a.H;
   const int hk = hh / a.group;                                  // K / V head
@@ -1060,6 +1071,10 @@ __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
     __syncthreads();
     U = meta[4];
   }
+
+  // This workgroup's part of the walk.
+  const int u0 = SPLIT ? static_cast<int>(static_cast<int64_t>(U) * split / a.splits) : 0;
+  const int u1 = SPLIT ? static_cast<int>(static_cast<int64_t>(U) * (split + 1) / a.splits) : U;
 
   // Staging (as in attn_fwd_kernel): wave w fetches its NI KB of K rows and
   // of the V^T tile of a block, one 1 KB buffer load each.
@@ -1195,14 +1210,14 @@ __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
       else
         return __builtin_amdgcn_readfirstlane(uni[u]);
     };
-    uint32_t e = ent(0);
+    uint32_t e = ent(u0);
     {
       const int j0 = static_cast<int>(e & TAG_BLOCK);
 #pragma unroll
       for (int part = 0; part < NDS; ++part) stage_part(j0, stage_k(0), stage_v(0), part);
     }
     auto step = [&](int u, auto par_tag) {
-      const uint32_t en = ent(u + 1 < U ? u + 1 : U - 1);  // the last step re-stages its own block
+      const uint32_t en = ent(u + 1 < u1 ? u + 1 : u1 - 1);  // the last step re-stages its own block
       const int j = static_cast<int>(e & TAG_BLOCK), jn = static_cast<int>(en & TAG_BLOCK);
       // vmcnt(0): this wave's staging of entry u landed; the barrier: every
       // wave's did, and the other stage is free. Written as one asm statement
@@ -1216,22 +1231,44 @@ __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
         entry_step(j, std::integral_constant<int, 2>{}, par_tag, fast_tag, jn, mset);
       e = en;
     };
-    for (int u = 0; u < U; u += 2) {
+    for (int u = u0; u < u1; u += 2) {
       step(u, std::integral_constant<int, 0>{});
-      if (u + 1 < U) step(u + 1, std::integral_constant<int, 1>{});
+      if (u + 1 < u1) step(u + 1, std::integral_constant<int, 1>{});
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last step's staging landed
   };
 
-  if (U > 0) {
-    walk(std::true_type{});
-    const bool bad = ballot64(!pair_sums_ok<HD>(st)) != 0;
+  if (u1 > u0) {
+    // A part whose first block hides keys from a query cannot take that
+    // query's maximum from it: the row check below then asks for the online
+    // walk, and that part starts with it.
+    const bool online = SPLIT && block_needs_mask(u0, irow[0], true, Nk, a.causal, a.qoff);
+    if (!online) walk(std::true_type{});
+    const bool bad = online || ballot64(!pair_sums_ok<HD>(st)) != 0;
     if (lane == 0) wave_bad[w] = bad ? 1 : 0;
     __syncthreads();
     if ((wave_bad[0] | wave_bad[1] | wave_bad[2] | wave_bad[3]) != 0) {
       pair_reset<HD>(st, c);
       walk(std::false_type{});
     }
+  }
+
+  if constexpr (SPLIT) {
+    // Each wave writes its own queries' partials.
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const int qtok = 64 * irow[r] + 16 * w + l16;
+      if (irow[r] >= M || qtok >= N) continue;
+      const int64_t x = (static_cast<int64_t>(split) * a.BH + bh) * N + qtok;
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt)
+        *reinterpret_cast<f32x4*>(a.po + x * HD + 16 * dt + 4 * g) = st.oacc[r][dt];
+      if (g == 0) {
+        a.pml[x] = st.m_run[r];
+        a.pml[static_cast<int64_t>(a.splits) * a.BH * N + x] = st.lacc[r][0];
+      }
+    }
+    return;
   }
 
   // Each wave writes its own queries: O = O^T / l, lse = (m c + log2 l) ln 2.
@@ -1252,6 +1289,39 @@ __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
       a.lse[static_cast<int64_t>(bh) * N + qtok] =
           l > 0.f ? (st.m_run[r] * c + __log2f(l)) * 0.69314718055994531f : -INFINITY;
   }
+}
+
+// Merges the splits of attn_pair_kernel<LIST_DENSE_SPLIT>: HD / 4 threads per
+// query, each four output values. A split in which the query has no key has
+// l = 0 and is skipped.
+template <bool BF16, int HD>
+__global__ __launch_bounds__(256) void split_combine_kernel(AttnArgs a) {
+  constexpr int TD = HD / 4;
+  const int64_t rows = static_cast<int64_t>(a.BH) * a.N;
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * (256 / TD) + threadIdx.x / TD;
+  if (row >= rows) return;
+  const int d4 = threadIdx.x % TD;
+  const float* pl = a.pml + a.splits * rows;
+  float m = M_EMPTY;
+  for (int s = 0; s < a.splits; ++s) m = fmaxf(m, a.pml[s * rows + row]);
+  float l = 0.f;
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int s = 0; s < a.splits; ++s) {
+    const float ls = pl[s * rows + row];
+    const float f = __builtin_amdgcn_exp2f((a.pml[s * rows + row] - m) * a.scale_log2);
+    const f32x4 x = reinterpret_cast<const f32x4*>(a.po + (s * rows + row) * HD)[d4];
+    if (ls > 0.f) {
+      l += ls * f;
+      o += x * f;
+    }
+  }
+  o *= l > 0.f ? 1.0f / l : 0.f;
+  const int64_t bh = row / a.N, t = row - bh * a.N, b = bh / a.H, hh = bh - b * a.H;
+  uint16_t* ob = static_cast<uint16_t*>(a.o) + b * a.os[0] + hh * a.os[1] + t * a.os[2];
+  *reinterpret_cast<u32x2*>(ob + 4 * d4) = u32x2{pack2<BF16>(o[0], o[1]), pack2<BF16>(o[2], o[3])};
+  if (a.lse && d4 == 0)
+    a.lse[row] = l > 0.f ? (m * a.scale_log2 + __log2f(l)) * 0.69314718055994531f : -INFINITY;
 }
 
 // ---------------------------------------------------------------------------
@@ -1576,8 +1646,15 @@ __global__ __launch_bounds__(64 * NW) void key_score_kernel(KeyScoreArgs a) {
   }
   const int key = j * BS + lane;
   if (has_keys && key < a.Nk) {
-    const float base = key < a.n_old ? a.old[b * a.olds[0] + hh * a.olds[1] + key] : 0.f;
-    a.score[b * a.ss[0] + hh * a.ss[1] + key] = base + mine;
+    // Where the totals go is read from the arguments here, through a pointer
+    // the compiler cannot look through: held in scalar registers over the
+    // loop, these spilled there (16384 causal queries, 32 heads, in the
+    // profiler: 1359 against 1318 us).
+    typedef __attribute__((address_space(4))) const KeyScoreArgs* args_ptr;
+    args_ptr pa = (args_ptr)__builtin_amdgcn_kernarg_segment_ptr();  // the one argument
+    asm volatile("" : "+s"(pa));
+    const float base = key < pa->n_old ? pa->old[b * pa->olds[0] + hh * pa->olds[1] + key] : 0.f;
+    pa->score[b * pa->ss[0] + hh * pa->ss[1] + key] = base + mine;
   }
 }
 
@@ -1734,7 +1811,8 @@ cab_status_t launch_attn(const char* fn, const void* q, const void* k, const voi
                          const int64_t* k_strides, const int64_t* o_strides,
                          const int32_t* kv_idx, const int32_t* kv_cnt, int32_t kmax, float scale,
                          int causal, void* out, float* lse, hipStream_t s,
-                         const uint64_t* submask = nullptr, int sub_shift = 0) {
+                         const uint64_t* submask = nullptr, int sub_shift = 0, int splits = 1,
+                         float* parts = nullptr) {
   const int64_t M = ceil_div(g.Nq, BS);
   AttnArgs a;
   a.q = q;
@@ -1762,13 +1840,22 @@ cab_status_t launch_attn(const char* fn, const void* q, const void* k, const voi
   a.causal = causal ? 1 : 0;
   a.submask = submask;
   a.sub_shift = sub_shift;
+  a.splits = splits;
+  a.po = parts;
+  a.pml = parts ? parts + static_cast<int64_t>(splits) * a.BH * a.N * g.D : nullptr;
   if (dtype != CAB_F32 && submask == nullptr && pair_enabled() &&
       ((g.list == LIST_LDS && kmax <= PAIR_KMAX) || g.list == LIST_DENSE)) {
     const dim3 pgrid(static_cast<unsigned>(g.B * g.H * ((M + 1) / 2)));
     auto go = [&](auto dt_tag, auto hd_tag) {
       constexpr cab_dtype_t DT = decltype(dt_tag)::value;
       constexpr int HD = decltype(hd_tag)::value;
-      if (g.list == LIST_DENSE)
+      if (g.list == LIST_DENSE && splits > 1) {
+        const dim3 sgrid(pgrid.x * static_cast<unsigned>(splits));
+        attn_pair_kernel<DT, LIST_DENSE_SPLIT, HD><<<sgrid, 256, 0, s>>>(a);
+        const int64_t per = 256 / (HD / 4);
+        split_combine_kernel<DT == CAB_BF16, HD>
+            <<<static_cast<unsigned>(ceil_div(static_cast<int64_t>(a.BH) * a.N, per)), 256, 0, s>>>(a);
+      } else if (g.list == LIST_DENSE)
         attn_pair_kernel<DT, LIST_DENSE, HD><<<pgrid, 256, 0, s>>>(a);
       else
         attn_pair_kernel<DT, LIST_LDS, HD><<<pgrid, 256, 0, s>>>(a);
@@ -2084,20 +2171,36 @@ cab_status_t check_score_rows(const char* fn, const void* q, const float* lse,
 // (fp32: K and V) and, when the totals need it and the caller keeps no lse,
 // the lse rows.
 struct DensePlan {
-  bool rows;        // the few-row kernels
-  size_t off_lse, bytes;
+  int splits;  // of the key blocks (16-bit inputs)
+  size_t off_lse, off_parts, bytes;
 };
+
+// Splits of the key blocks that fill the chip's 512 workgroup slots (two per
+// CU) when the query pairs alone do not. Each part holds at least ten blocks
+// on (the causal) average: 40 queries of 32 heads against 5000 keys ran 77.5 us
+// whole and 32.5 us in eight parts, but 1000 against their own 1000 keys 27.5 us
+// whole and 37 us in two, where writing and merging the partials costs more.
+int dense_splits(cab_dtype_t dtype, int64_t B, int64_t H, int64_t N_q, int64_t N_k) {
+  if (dtype == CAB_F32 || !pair_enabled()) return 1;
+  const int64_t wgs = B * H * ceil_div(N_q, 2 * BS);
+  const int64_t fill = 512 / wgs, parts = (2 * ceil_div(N_k, BS) - ceil_div(N_q, BS)) / 20;
+  const int64_t n = fill < parts ? fill : parts;
+  return static_cast<int>(n < 1 ? 1 : n > 8 ? 8 : n);
+}
 DensePlan dense_plan(cab_dtype_t dtype, int64_t B, int64_t H, int64_t H_kv, int64_t N_q,
                      int64_t N_k, int64_t D, bool rows, bool scores) {
   DensePlan p;
-  p.rows = rows;
-  p.off_lse = 0;
+  p.splits = 1;
+  p.off_lse = p.off_parts = 0;
   if (rows) {
     p.bytes = row_attn_workspace(B, H, H_kv, N_q, N_k, D, scores);
     return p;
   }
   p.off_lse = dense_packed_bytes(dtype, B, H_kv, N_k, D);
-  p.bytes = p.off_lse + (scores ? static_cast<size_t>(B * H * N_q) * 4 : 0);
+  p.off_parts = p.off_lse + (scores ? static_cast<size_t>(round_up(B * H * N_q, 4)) * 4 : 0);
+  p.bytes = p.off_parts;
+  p.splits = dense_splits(dtype, B, H, N_q, N_k);
+  if (p.splits > 1) p.bytes += static_cast<size_t>(p.splits * B * H * N_q * (D + 2)) * 4;
   return p;
 }
 
@@ -2133,7 +2236,7 @@ cab_status_t dense_forward(const char* fn, const void* q, const void* k, const v
               "%s: workspace of %zu bytes given, %zu needed", fn, workspace_bytes, least);
   CAB_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16 == 0, CAB_EWORKSPACE,
               "%s: workspace not 16-byte aligned", fn);
-  if (row_attn_applies(dtype, B, H, H_kv, N_q, N_k, D, k_strides, v_strides) &&
+  if (row_attn_applies(dtype, B, H, H_kv, N_q, N_k, D, k_strides, v_strides, scores) &&
       workspace_bytes >= dense_plan(dtype, B, H, H_kv, N_q, N_k, D, true, scores).bytes) {
     RowAttnProblem p{};
     p.dtype = dtype;
@@ -2156,9 +2259,10 @@ cab_status_t dense_forward(const char* fn, const void* q, const void* k, const v
     }
     return row_attn_launch(fn, p, workspace, s);
   }
-  const DensePlan plan = dense_plan(dtype, B, H, H_kv, N_q, N_k, D, false, scores && !lse);
-  CAB_REQUIRE(workspace_bytes >= plan.bytes, CAB_EWORKSPACE,
-              "%s: workspace of %zu bytes given, %zu needed", fn, workspace_bytes, plan.bytes);
+  DensePlan plan = dense_plan(dtype, B, H, H_kv, N_q, N_k, D, false, scores && !lse);
+  CAB_REQUIRE(workspace_bytes >= plan.off_parts, CAB_EWORKSPACE,
+              "%s: workspace of %zu bytes given, %zu needed", fn, workspace_bytes, plan.off_parts);
+  if (workspace_bytes < plan.bytes) plan.splits = 1;  // no room for partials
   if (scores && !lse)
     lse = reinterpret_cast<float*>(static_cast<char*>(workspace) + plan.off_lse);
   if (scores && (st = check_score_rows(fn, q, lse, q_strides, esize)) != CAB_OK) return st;
@@ -2169,7 +2273,9 @@ cab_status_t dense_forward(const char* fn, const void* q, const void* k, const v
   if (st != CAB_OK) return st;
   const AttnGeom g{B, H, H_kv, N_q, N_k, D, N_k - N_q, LIST_DENSE};
   st = launch_attn(fn, q, k, workspace, dtype, g, q_strides, k_strides, o_strides, nullptr,
-                   nullptr, 1, scale, causal, out, lse, s);
+                   nullptr, 1, scale, causal, out, lse, s, nullptr, 0, plan.splits,
+                   plan.splits > 1 ? reinterpret_cast<float*>(static_cast<char*>(workspace) + plan.off_parts)
+                                   : nullptr);
   if (st != CAB_OK || !scores) return st;
   return launch_key_scores(fn, q, k, lse, dtype, B, H, H_kv, N_q, N_k, D, q_strides, k_strides,
                            scale, causal, t, s);
@@ -2192,7 +2298,7 @@ extern "C" size_t cab_flash_attn_scores_workspace_bytes(cab_dtype_t dtype, int64
   if (B <= 0 || H <= 0 || H_kv <= 0 || H % H_kv != 0 || N_q <= 0 || N_k <= 0 ||
       (D != 64 && D != 128) || !k_strides || !v_strides)
     return 0;
-  const bool rows = row_attn_applies(dtype, B, H, H_kv, N_q, N_k, D, k_strides, v_strides);
+  const bool rows = row_attn_applies(dtype, B, H, H_kv, N_q, N_k, D, k_strides, v_strides, scores != 0);
   return dense_plan(dtype, B, H, H_kv, N_q, N_k, D, rows, scores != 0).bytes;
 }
 

@@ -302,7 +302,7 @@ cab_status_t cab_attn_key_scores(const void* q, const void* k, const float* lse,
  * (nothing is added to) and may be scores itself. workspace:
  * cab_flash_attn_scores_workspace_bytes() bytes for the same sizes and
  * strides (scores != 0 when totals are asked for), 16-byte aligned,
- * overwritten. At most 64 rows per K / V head (H / H_kv * N_q; decode steps
+ * overwritten. At most 32 rows per K / V head (H / H_kv * N_q; decode steps
  * and short chunks) run kernels that split the key range over the chip and
  * read K and V once; so does cab_flash_attn_fwd when its workspace holds
  * that path's partials.

@@ -1,9 +1,10 @@
 """Dense attention for few query rows (decode steps, short chunks) with the
 key totals in the same call: cab_flash_attn_scores_fwd at the edges of the
-key split (32-key steps, four per workgroup), of the row tiles (16, 32 and 64
-rows per K / V head, and 65, which runs the general kernels), and of the
-running totals (none, shorter, as long as the keys), against the float64
-oracle; and cab_flash_attn_fwd with a workspace the partials do not fit."""
+key split (32-key steps, four per workgroup), of the row tiles (16 and 32
+rows per K / V head, and 33, which runs the general kernels), of the general
+kernels' own split over the keys, and of the running totals (none, shorter,
+as long as the keys), against the float64 oracle; and cab_flash_attn_fwd with
+a workspace the partials do not fit."""
 
 import math
 
@@ -42,10 +43,12 @@ CASES = [  # (B, H, H_kv, N_q, N_k)
     (1, 4, 4, 16, 500),      # a full row tile
     (1, 4, 4, 17, 1025),     # one row into the second; one key past a totals chunk
     (2, 8, 2, 8, 1000),      # 32 rows
-    (1, 4, 1, 9, 2047),      # 36 rows: four tiles, two of them partly or wholly empty
-    (1, 32, 4, 8, 4099),     # 64 rows
-    (1, 5, 1, 13, 700),      # 65 rows: the general kernels
-    (1, 2, 1, 20, 7),        # more queries than keys (causal: the first see none)
+    (1, 32, 4, 3, 4099),     # 24 rows: the second tile half empty
+    (1, 3, 1, 11, 700),      # 33 rows: the general kernels
+    (1, 2, 1, 16, 7),        # more queries than keys (causal: the first see none)
+    (1, 4, 2, 33, 1250),     # general kernels, keys split in two
+    (1, 4, 4, 130, 2100),    # three parts, the last one past the first queries' keys
+    (1, 2, 2, 40, 6000),     # eight parts, the most
 ]
 
 
@@ -94,11 +97,12 @@ def test_masked_values_and_far_maxima(cuda):
 
 @pytest.mark.parametrize("dt", ["bf16", "fp32"])
 def test_flash_fwd_workspace_decides_the_path(cuda, dt):
-    """cab_flash_attn_fwd takes its documented workspace whatever path runs: 64
-    rows over 64 keys have partials larger than the packed block, so the
-    general kernels run there; with a larger workspace the few-row ones do."""
+    """cab_flash_attn_fwd takes its documented workspace whatever path runs: for
+    16-bit inputs the partials of 32 rows over 64 keys are larger than the
+    packed block, so the general kernels run there; with a larger workspace
+    the few-row ones do."""
     lib = nat.load()
-    B, H, Hkv, Nq, Nk, D = 1, 64, 1, 1, 64, 128
+    B, H, Hkv, Nq, Nk, D = 1, 32, 1, 1, 64, 128
     q = seeded((B, H, Nq, D), 5, DTYPES[dt]).to(cuda)
     k = seeded((B, Hkv, Nk, D), 6, DTYPES[dt]).to(cuda)
     v = seeded((B, Hkv, Nk, D), 7, DTYPES[dt]).to(cuda)
