@@ -377,16 +377,30 @@ __device__ __forceinline__ bool block_needs_mask(int j, int i, bool valid, int N
   return !valid || (j + 1) * BS > Nk || (causal && j * BS + BS - 1 > i * BS + qoff);
 }
 
+// The kept sub-tiles of wave (kh, qh)'s 32 x 32 quadrant of a 64 x 64 tile with
+// sub-tile mask sm (AttnArgs::submask): bit (q / bs) (32 / bs) + k / bs for
+// query q and key k of the quadrant; QUAD_FULL when every one is kept.
+constexpr uint32_t QUAD_FULL = ~0u;
+__device__ __forceinline__ uint32_t quadrant_bits(uint64_t sm, int kh, int qh, int sub_shift) {
+  const int n = 32 >> sub_shift, width = 2 * n;  // sub-tiles per quadrant and tile side
+  const uint32_t line = (1u << n) - 1u;
+  uint32_t q = 0;
+  for (int u = 0; u < n; ++u)
+    q |= (static_cast<uint32_t>(sm >> ((n * qh + u) * width + n * kh)) & line) << (u * n);
+  return q == static_cast<uint32_t>((uint64_t{1} << (n * n)) - 1) ? QUAD_FULL : q;
+}
+
 // One key block j (staged at ks / vts) for the wave's queries of query block i:
 //   S^T = K_kh Q^T (16 MFMA), masks, online softmax (fp32, log2 domain),
 //   O^T += V_kh^T P^T (16 MFMA), row sums = 1 P^T (2 MFMA).
 // fp32 (split operands, the lo halves 16 KB past the hi ones in LDS):
 // 48 + 48 + 4 MFMA. Keys at or past Nk and (causal) keys after t + qoff for
-// query t are dropped.
-template <cab_dtype_t DT, int HD, int SM, typename Stager>
+// query t are dropped. quad: the kept sub-tiles of the wave's 32 x 32 quadrant
+// (quadrant_bits; QUAD_FULL when none is dropped).
+template <cab_dtype_t DT, int HD, int SM, bool SUB, typename Stager>
 __device__ __forceinline__ void acc_block(WaveAcc<HD>& s, const WaveGeo<HD>& ge, const char* ks,
                                           const u32x4* vts, int j, int i, bool valid, int Nk,
-                                          bool causal, int qoff, float c, uint64_t sm,
+                                          bool causal, int qoff, float c, uint32_t quad,
                                           int sub_shift, const Stager& stg) {
   using G = Dims<HD>;
   constexpr int NDS = G::NDS, NDT = G::NDT;
@@ -438,22 +452,22 @@ __device__ __forceinline__ void acc_block(WaveAcc<HD>& s, const WaveGeo<HD>& ge,
     }
   }
 
-  const bool subm = sm != ~0ull;  // a tile of smaller blocks, some of them dropped
+  const bool subm = SUB && quad != QUAD_FULL;  // some sub-tiles dropped
   if (block_needs_mask(j, i, valid, Nk, causal, qoff) || subm) {
 #pragma unroll
     for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-      for (int qt = 0; qt < 2; ++qt)
+      for (int qt = 0; qt < 2; ++qt) {
+        const int kl = 16 * tt + 4 * ge.g, ql = 16 * qt + ge.l16;  // in the quadrant; keys kl .. + 3
+        // (sub-tiles are at least 8 keys wide: one bit for the four)
+        const bool gone = subm && ((quad >> (((ql >> sub_shift) << (5 - sub_shift)) |
+                                             (kl >> sub_shift))) & 1u) == 0;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int kl = 32 * ge.kh + 16 * tt + 4 * ge.g + r, ql = 32 * ge.qh + 16 * qt + ge.l16;
-          const int ktok = j * BS + kl, qtok = i * BS + ql;
-          bool drop = !valid || ktok >= Nk || (causal && ktok > qtok + qoff);
-          if (subm)
-            drop = drop || ((sm >> (((ql >> sub_shift) << (6 - sub_shift)) | (kl >> sub_shift))) &
-                            1ull) == 0;
-          if (drop) sc[tt][qt][r] = -INFINITY;
+          const int ktok = j * BS + 32 * ge.kh + kl + r, qtok = i * BS + 32 * ge.qh + ql;
+          if (gone || !valid || ktok >= Nk || (causal && ktok > qtok + qoff)) sc[tt][qt][r] = -INFINITY;
         }
+      }
   }
   float mx[2];
   if constexpr (SM != SM_FIXED) {
@@ -621,7 +635,8 @@ __device__ __forceinline__ uint32_t k_lane_off(int group, int lane, int64_t krow
 // blocks, merged by split_combine_kernel.
 constexpr int LIST_LDS = 0, LIST_GLOBAL = 1, LIST_DENSE = 2, LIST_DENSE_SPLIT = 3;
 
-template <cab_dtype_t DT, int LIST, int HD>
+// SUB: the entries carry sub-tile masks (block sizes below 64).
+template <cab_dtype_t DT, int LIST, int HD, bool SUB>
 __global__ __launch_bounds__(256, DT == CAB_F32 ? 1 : 2) void attn_fwd_kernel(AttnArgs a) {
   using G = Dims<HD>;
   constexpr bool SPLIT = DT == CAB_F32;
@@ -737,6 +752,10 @@ __global__ __launch_bounds__(256, DT == CAB_F32 ? 1 : 2) void attn_fwd_kernel(At
   acc_init<DT, HD>(st, ge, qb, a.qs[2], i * BS + 32 * ge.qh, N, c);
   __shared__ int wave_bad[4];
   auto block_of = [&](int j) { return (j >= 0 && j < Mk) ? j : 0; };
+  const uint64_t* smask = SUB ? a.submask + (static_cast<int64_t>(bh) * M + i) * a.kmax : nullptr;
+  auto uniform = [](uint32_t x) {
+    return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(x)));
+  };
 
   // One walk over the row's blocks. FAST: the first block sets each query's
   // maximum and the rest use it unchanged (SM_FIRST, then SM_FIXED);
@@ -744,6 +763,8 @@ __global__ __launch_bounds__(256, DT == CAB_F32 ? 1 : 2) void attn_fwd_kernel(At
   auto walk = [&](auto fast_tag) {
     constexpr bool FAST = decltype(fast_tag)::value;
     int jraw = entry(0);
+    uint64_t smraw = 0;
+    if constexpr (SUB) smraw = smask[0];
     stage(block_of(jraw), stage_k(0), stage_v(0));
     acc_q_ready<DT, HD>(st);
 
@@ -754,26 +775,35 @@ __global__ __launch_bounds__(256, DT == CAB_F32 ? 1 : 2) void attn_fwd_kernel(At
       constexpr int SM = decltype(sm_tag)::value;
       const bool valid = jraw >= 0 && jraw < Mk;
       const int j = valid ? jraw : 0;
-      const uint64_t sm = a.submask ? a.submask[(static_cast<int64_t>(bh) * M + i) * a.kmax + p]
-                                    : ~0ull;
+      const uint32_t quad = SUB
+                                ? quadrant_bits(static_cast<uint64_t>(uniform(static_cast<uint32_t>(smraw))) |
+                                                    static_cast<uint64_t>(uniform(static_cast<uint32_t>(smraw >> 32))) << 32,
+                                                ge.kh, ge.qh, a.sub_shift)
+                                : QUAD_FULL;
       __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's staging of block p landed
       __builtin_amdgcn_s_barrier();        // ... and every wave's; stage PAR ^ 1 is free
       int jnext = 0;
-      if constexpr (SPLIT) {
+      // The next entry's mask, waited for with its staging.
+      if constexpr (SUB) smraw = smask[p + 1 < cnt ? p + 1 : p];
+      if constexpr (SPLIT || SUB) {
         if (p + 1 < cnt) {
           jnext = entry(p + 1);
           stage(block_of(jnext), stage_k(PAR ^ 1), stage_v(PAR ^ 1));
         }
-        acc_block<DT, HD, SM>(st, ge, reinterpret_cast<const char*>(stage_k(PAR)), stage_v(PAR),
-                              j, i, valid, Nk, a.causal, a.qoff, c, sm, a.sub_shift, [](int) {});
+        // A quadrant without kept sub-tiles is skipped. (Staging first, so that the
+        // branch has one side: with the loads in both sides the accumulators
+        // were copied and spilled.)
+        if (!SUB || quad != 0u)
+          acc_block<DT, HD, SM, SUB>(st, ge, reinterpret_cast<const char*>(stage_k(PAR)), stage_v(PAR),
+                              j, i, valid, Nk, a.causal, a.qoff, c, quad, a.sub_shift, [](int) {});
       } else {
         // unconditional (the last step re-stages a valid block into the free
         // stage; waited for after the loop) so that the loads sit between the MFMAs
         const int e = entry(p + 1 < cnt ? p + 1 : cnt - 1);
         jnext = p + 1 < cnt ? e : 0;
         const int js = block_of(jnext);
-        acc_block<DT, HD, SM>(st, ge, reinterpret_cast<const char*>(stage_k(PAR)), stage_v(PAR),
-                              j, i, valid, Nk, a.causal, a.qoff, c, sm, a.sub_shift,
+        acc_block<DT, HD, SM, SUB>(st, ge, reinterpret_cast<const char*>(stage_k(PAR)), stage_v(PAR),
+                              j, i, valid, Nk, a.causal, a.qoff, c, quad, a.sub_shift,
                               [&](int ds) { stage_part(js, stage_k(PAR ^ 1), stage_v(PAR ^ 1), ds); });
       }
       jraw = jnext;
@@ -796,15 +826,19 @@ __global__ __launch_bounds__(256, DT == CAB_F32 ? 1 : 2) void attn_fwd_kernel(At
   };
 
   if (cnt > 0) {
-    walk(std::true_type{});
+    // With sub-tile masks a query often has no key in the row's first tile, so
+    // that walk takes the online softmax at once (24 heads of 5003 tokens,
+    // block size 32, D = 64: the fixed-maximum walk failed and every row was
+    // walked twice, 303 us).
+    if constexpr (!SUB) walk(std::true_type{});
     // Every wave reports whether its fixed-maximum state is usable; if any
     // is not, the whole row is walked again with the online softmax (the
     // barrier also frees both stages for that walk's first loads).
-    const bool bad = __builtin_amdgcn_ballot_w64(!row_sums_ok<HD>(st)) != 0;
+    const bool bad = SUB || __builtin_amdgcn_ballot_w64(!row_sums_ok<HD>(st)) != 0;
     if (threadIdx.x % 64 == 0) wave_bad[w] = bad ? 1 : 0;
     __syncthreads();
     if ((wave_bad[0] | wave_bad[1] | wave_bad[2] | wave_bad[3]) != 0) {
-      acc_reset<HD>(st, c);
+      if constexpr (!SUB) acc_reset<HD>(st, c);
       walk(std::false_type{});
     }
   }
@@ -1333,10 +1367,11 @@ __global__ __launch_bounds__(256) void split_combine_kernel(AttnArgs a) {
 //    which the executors skip).
 //  relist_merge_kernel (bs = 64 / r): the r bs-rows of a 64-row give their
 //    entries jb as (tile jb / r, sub-tile bit u r + jb % r) for sub-row u.
-//    One wave merges them in list order: a pair joins the first entry of
-//    its tile that lacks its bit, or starts a new entry. A block listed
-//    twice therefore counts twice, as in the caller's lists. Each entry
-//    carries its 64-bit sub-tile mask (AttnArgs::submask).
+//    Lists without repeats (and at most MERGE_TILES_MAX tiles) are merged
+//    through one mask per tile; others by one wave in list order: a pair
+//    joins the first entry of its tile that lacks its bit, or starts a new
+//    entry. A block listed twice therefore counts twice, as in the caller's
+//    lists. Each entry carries its 64-bit sub-tile mask (AttnArgs::submask).
 // ---------------------------------------------------------------------------
 struct RelistArgs {
   const int32_t* idx;  // [BH, Mb, kmax]
@@ -1345,6 +1380,7 @@ struct RelistArgs {
   int32_t* cnt64;      // [BH, M64]
   uint64_t* sub64;     // [BH, M64, K64] (merge only)
   int32_t Mb, M64, Mk64, kmax, K64, r;
+  int tile_map;  // merge: the masks of all Mk64 tiles fit the LDS
 };
 
 __global__ __launch_bounds__(64) void relist_expand_kernel(RelistArgs a) {
@@ -1365,11 +1401,51 @@ __global__ __launch_bounds__(64) void relist_expand_kernel(RelistArgs a) {
 
 __global__ __launch_bounds__(64) void relist_merge_kernel(RelistArgs a) {
   extern __shared__ __align__(16) unsigned char relist_lds[];
-  uint64_t* lsub = reinterpret_cast<uint64_t*>(relist_lds);        // [K64]
-  int32_t* lidx = reinterpret_cast<int32_t*>(lsub + a.K64);         // [K64]
   const int64_t row = blockIdx.x;
   const int64_t bh = row / a.M64, i64 = row - bh * a.M64;
   const int lane = lane_id();
+  if (a.tile_map) {
+    // Lists without repeats (the usual ones): every pair sets its bit in its
+    // tile's mask, 64 at a time, and the tiles with bits are the entries, in
+    // tile order. A repeated block is seen by its bit being set already.
+    unsigned long long* tile = reinterpret_cast<unsigned long long*>(relist_lds);  // [Mk64]
+    for (int t = lane; t < a.Mk64; t += 64) tile[t] = 0;
+    __syncthreads();
+    bool repeat = false;
+    for (int u = 0; u < a.r; ++u) {
+      const int64_t ib = i64 * a.r + u;
+      if (ib >= a.Mb) break;
+      int cnt = a.cnt[bh * a.Mb + ib];
+      cnt = cnt < 0 ? 0 : (cnt > a.kmax ? a.kmax : cnt);
+      const int32_t* src = a.idx + (bh * a.Mb + ib) * a.kmax;
+      for (int e = lane; e < cnt; e += 64) {
+        const int jb = src[e];
+        if (jb < 0 || jb >= a.Mb) continue;
+        const unsigned long long bit = 1ull << (u * a.r + jb % a.r);
+        repeat = repeat || (atomicOr(&tile[jb / a.r], bit) & bit) != 0;
+      }
+    }
+    __syncthreads();
+    if (ballot64(repeat) == 0) {
+      int n = 0;
+      for (int base = 0; base < a.Mk64; base += 64) {
+        const int t = base + lane;
+        const unsigned long long m = t < a.Mk64 ? tile[t] : 0ull;
+        const uint64_t has = ballot64(m != 0);
+        if (m != 0) {
+          const int64_t at = row * a.K64 + n + static_cast<int>(rank_below64(has));
+          a.idx64[at] = t;
+          a.sub64[at] = m;
+        }
+        n += __popcll(has);
+      }
+      if (lane == 0) a.cnt64[row] = n;
+      return;
+    }
+    __syncthreads();  // the LDS is used anew below
+  }
+  uint64_t* lsub = reinterpret_cast<uint64_t*>(relist_lds);        // [K64]
+  int32_t* lidx = reinterpret_cast<int32_t*>(lsub + a.K64);         // [K64]
   int n = 0;  // entries so far (uniform)
   for (int u = 0; u < a.r; ++u) {
     const int64_t ib = i64 * a.r + u;
@@ -1672,6 +1748,7 @@ namespace {
 bool executor_block_size(int64_t bs) {
   return bs == 8 || bs == 16 || bs == 32 || bs == 64 || bs == 128 || bs == 256;
 }
+constexpr int64_t MERGE_TILES_MAX = 4096;  // key tiles whose masks the merge holds (32 KB of LDS)
 constexpr int64_t MERGE_K64_MAX = 4096;  // merged 64-tile entries per row (LDS of the merge)
 
 cab_status_t check_common(const char* fn, cab_dtype_t dtype, int64_t B, int64_t H, int64_t N,
@@ -1790,12 +1867,16 @@ bool pair_enabled() {
 
 template <cab_dtype_t DT, int HD>
 void launch_attn_kernel(int list, dim3 grid, hipStream_t s, const AttnArgs& a) {
-  if (list == LIST_LDS)
-    attn_fwd_kernel<DT, LIST_LDS, HD><<<grid, 256, 0, s>>>(a);
+  if (a.submask && list == LIST_LDS)
+    attn_fwd_kernel<DT, LIST_LDS, HD, true><<<grid, 256, 0, s>>>(a);
+  else if (a.submask)
+    attn_fwd_kernel<DT, LIST_GLOBAL, HD, true><<<grid, 256, 0, s>>>(a);
+  else if (list == LIST_LDS)
+    attn_fwd_kernel<DT, LIST_LDS, HD, false><<<grid, 256, 0, s>>>(a);
   else if (list == LIST_GLOBAL)
-    attn_fwd_kernel<DT, LIST_GLOBAL, HD><<<grid, 256, 0, s>>>(a);
+    attn_fwd_kernel<DT, LIST_GLOBAL, HD, false><<<grid, 256, 0, s>>>(a);
   else
-    attn_fwd_kernel<DT, LIST_DENSE, HD><<<grid, 256, 0, s>>>(a);
+    attn_fwd_kernel<DT, LIST_DENSE, HD, false><<<grid, 256, 0, s>>>(a);
 }
 
 // Problem geometry of one executor call: query heads H over Hkv K / V heads,
@@ -2029,11 +2110,15 @@ extern "C" cab_status_t cab_block_sparse_attn_fwd(
     ra.kmax = kmax;
     ra.K64 = static_cast<int32_t>(tl.K64);
     ra.r = static_cast<int32_t>(tl.r);
+    ra.tile_map = 0;
     const dim3 rgrid(static_cast<unsigned>(B * H * tl.M64));
     if (block_size > BS) {
       relist_expand_kernel<<<rgrid, 64, 0, s>>>(ra);
     } else {
-      const size_t lds = static_cast<size_t>(tl.K64) * 12;
+      ra.tile_map = tl.M64 <= MERGE_TILES_MAX;
+      const size_t lists = static_cast<size_t>(tl.K64) * 12;
+      const size_t tiles = ra.tile_map ? static_cast<size_t>(tl.M64) * 8 : 0;
+      const size_t lds = lists > tiles ? lists : tiles;
       relist_merge_kernel<<<rgrid, 64, lds, s>>>(ra);
     }
     if ((st = launch_status("cab_block_sparse_attn_fwd/relist")) != CAB_OK) return st;
