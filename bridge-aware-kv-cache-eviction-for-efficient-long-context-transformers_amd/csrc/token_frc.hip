@@ -189,7 +189,7 @@ constexpr int GRAM_ROWS = 32 * GRAM_WAVES;   // rows per workgroup
 struct KeyLayout {
   int64_t Np, dk, rb, tiles;  // padded rows, k-steps, 256-row blocks, 32-column tiles
   int64_t col_tiles, cs, wgs;  // tiles per workgroup, most splits of a row block, workgroups
-  size_t off_hi, off_lo, off_r, off_s, off_part, off_cpart, total;
+  size_t off_hi, off_lo, off_r, off_s, off_part, off_cpart, off_flag, total;
 };
 
 // Column splits of row block x: its tiles run from 8 x (the diagonal block)
@@ -231,6 +231,7 @@ KeyLayout key_layout(int64_t N, int64_t D) {
   L.off_s = take(static_cast<size_t>(L.Np) * 4);
   L.off_part = take(static_cast<size_t>(L.cs) * L.Np * 4);
   L.off_cpart = take(static_cast<size_t>(L.rb) * L.Np * 4);
+  L.off_flag = take(4);
   L.total = o;
   return L;
 }
@@ -241,69 +242,104 @@ struct PrepArgs {
   int64_t st[4];
   u32x4* hi;
   u32x4* lo;
+  int32_t* flag;  // cleared here; see GramArgs
 };
 
-// One wave per position: lane l (l < 32) owns dims 8 (l % 32) .. + 7, and
-// the two lane halves sum the even and odd (b, h) slices. VEC: unit dim
-// stride and 16-byte aligned rows, so a lane's dims are one or two 16-byte
-// loads per slice.
-template <typename T, bool VEC>
+// One wave per position: lane l owns dims 8 (l % DL) .. + 7 (DL = 8, 16 or 32
+// lanes hold D dims), and the 64 / DL lane groups sum every 64 / DL-th (b, h)
+// slice, so that no lane idles at D <= 128 and a wave's slices load together.
+// VEC: unit dim stride and 16-byte aligned rows, so a lane's dims are one or
+// two 16-byte loads per slice. 8192 positions of 8 heads, D = 128, bf16: 12.1 us
+// in the profiler (13.3 with 32 lanes a position); launch and load latency bound it.
+template <typename T, bool VEC, int DL>
 __global__ __launch_bounds__(256) void keys_prep_kernel(PrepArgs a) {
+  constexpr int SL = 64 / DL;  // slices summed side by side
+  if (blockIdx.x == 0 && threadIdx.x == 0) *a.flag = 0;
   const int64_t n = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   if (n >= a.Np) return;
-  const int lane = lane_id(), g = lane & 31, par = lane >> 5;
+  const int lane = lane_id(), g = lane % DL, par = lane / DL;
   float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (n < a.N) {
-    const T* base = static_cast<const T*>(a.k);
-    for (int64_t bh = par; bh < a.bh; bh += 2) {
-      const int64_t b = bh / a.H, h = bh - (bh / a.H) * a.H;
-      const T* p = base + b * a.st[0] + h * a.st[1] + n * a.st[2];
-      if constexpr (VEC) {
-        if (8 * g < a.D) {  // D % 8 == 0 on this path
-          float v[8];
-          if constexpr (sizeof(T) == 4) {
-            ld_vec<T>(p + 8 * g, v);
-            ld_vec<T>(p + 8 * g + 4, v + 4);
-          } else {
-            ld_vec<T>(p + 8 * g, v);
+    const T* base = static_cast<const T*>(a.k) + n * a.st[2];
+    const uint32_t H = static_cast<uint32_t>(a.H), slices = static_cast<uint32_t>(a.bh);
+    // Four slices of a lane are loaded before any is added.
+    constexpr int U = 4;
+    for (uint32_t bh0 = par; bh0 < slices; bh0 += U * SL) {
+      float v[U][8];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const uint32_t bh = bh0 + u * SL;
+        const uint32_t b = bh / H, h = bh - b * H;
+        const T* p = base + b * a.st[0] + h * a.st[1];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[u][e] = 0.f;
+        if constexpr (VEC) {
+          if (bh < slices && 8 * g < a.D) {  // D % 8 == 0 on this path
+            ld_vec<T>(p + 8 * g, v[u]);
+            if constexpr (sizeof(T) == 4) ld_vec<T>(p + 8 * g + 4, v[u] + 4);
           }
+        } else {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) x[e] += v[e];
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int64_t d = 8 * g + e;
-          if (d < a.D) x[e] += ld_elem<T>(p + d * a.st[3]);
+          for (int e = 0; e < 8; ++e) {
+            const int64_t d = 8 * g + e;
+            if (bh < slices && d < a.D) v[u][e] = ld_elem<T>(p + d * a.st[3]);
+          }
         }
       }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] += v[u][e];
     }
   }
+  // The groups add their slices by halves: each step a lane keeps one half of
+  // its dims and hands the other to its partner, so that it ends with 8 / SL
+  // dims of its own to normalise and split.
+  constexpr int ND = 8 / SL;
+#pragma unroll
+  for (int off = 32, half = 4; off >= DL; off >>= 1, half >>= 1) {
+    const bool up = (lane & off) != 0;
+#pragma unroll
+    for (int e = 0; e < half; ++e) {
+      const float mine = up ? x[half + e] : x[e], other = up ? x[e] : x[half + e];
+      x[e] = mine + shfl_xor_f32(other, off);
+    }
+  }
+  int d0 = 0;  // this lane's first dim of the eight
+#pragma unroll
+  for (int off = 32, half = 4; off >= DL; off >>= 1, half >>= 1) d0 += (lane & off) ? half : 0;
   const float cnt = static_cast<float>(a.bh);
   float ss = 0.f;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    x[e] += __shfl_xor(x[e], 32, 64);
+  for (int e = 0; e < ND; ++e) {
     x[e] = x[e] / cnt;
     ss = fmaf(x[e], x[e], ss);
   }
 #pragma unroll
-  for (int off = 16; off >= 1; off >>= 1) ss += shfl_xor_f32(ss, off);
+  for (int off = 32; off >= 1; off >>= 1) ss += shfl_xor_f32(ss, off);
   const float den = fmaxf(sqrtf(ss), 1e-12f);
-  if (par == 0 && g < 2 * a.dk) {
-    u32x4 h4, l4;
+  uint16_t hv[ND], lv[ND];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const float v0 = x[2 * q] / den, v1 = x[2 * q + 1] / den;
-      const uint16_t h0 = f32_to_bf16(v0), h1 = f32_to_bf16(v1);
-      const uint16_t l0 = f32_to_bf16(v0 - bf16_to_f32(h0)), l1 = f32_to_bf16(v1 - bf16_to_f32(h1));
-      h4[q] = static_cast<uint32_t>(h0) | (static_cast<uint32_t>(h1) << 16);
-      l4[q] = static_cast<uint32_t>(l0) | (static_cast<uint32_t>(l1) << 16);
-    }
-    const int64_t s = g >> 1, hh = g & 1;
-    const int64_t idx = ((n >> 5) * a.dk + s) * 64 + (n & 31) + 32 * hh;
-    a.hi[idx] = h4;
-    a.lo[idx] = l4;
+  for (int e = 0; e < ND; ++e) {
+    const float v = x[e] / den;
+    hv[e] = f32_to_bf16(v);
+    lv[e] = f32_to_bf16(v - bf16_to_f32(hv[e]));
+  }
+  const int64_t s = g >> 1, hh = g & 1;
+  const int64_t idx = (((n >> 5) * a.dk + s) * 64 + (n & 31) + 32 * hh) * 8 + d0;
+  uint16_t* ph = reinterpret_cast<uint16_t*>(a.hi) + idx;
+  uint16_t* pl = reinterpret_cast<uint16_t*>(a.lo) + idx;
+  if constexpr (ND == 1) {
+    *ph = hv[0];
+    *pl = lv[0];
+  } else if constexpr (ND == 2) {
+    *reinterpret_cast<uint32_t*>(ph) = hv[0] | static_cast<uint32_t>(hv[1]) << 16;
+    *reinterpret_cast<uint32_t*>(pl) = lv[0] | static_cast<uint32_t>(lv[1]) << 16;
+  } else {
+    *reinterpret_cast<u32x2*>(ph) = u32x2{hv[0] | static_cast<uint32_t>(hv[1]) << 16,
+                                          hv[2] | static_cast<uint32_t>(hv[3]) << 16};
+    *reinterpret_cast<u32x2*>(pl) = u32x2{lv[0] | static_cast<uint32_t>(lv[1]) << 16,
+                                          lv[2] | static_cast<uint32_t>(lv[3]) << 16};
   }
 }
 
@@ -313,6 +349,11 @@ struct GramArgs {
   const float* w;  // pass 1: S (zero past N)
   float* part;     // [cs][Np] row partials per column split
   float* cpart;    // [Np][rb] column partials per row block (columns right of its diagonal block)
+  // Set by the first pass's finalize when some weight S_j = r_j / (r_j + 1e-8) is
+  // not 1 in fp32 (a key of norm 0, or values that are not finite). Else pass
+  // 1 would form the sums of pass 0 again, bit for bit: it leaves at once
+  // (8192 positions, D = 128: 95.8 -> 46.2 us a call with it).
+  const int32_t* flag;
   int64_t Np, tiles, col_tiles, rb;
 };
 
@@ -341,6 +382,7 @@ __global__ __launch_bounds__(64 * GRAM_WAVES) void gram_kernel(GramArgs a) {
   static_assert(NDMA < 16, "vmcnt immediate");
   __shared__ __attribute__((aligned(16))) char ring[GRAM_STAGES * STAGE_BYTES];
   __shared__ float cbuf[GRAM_STAGES][GRAM_WAVES][32];
+  if (PASS == 1 && *a.flag == 0) return;
   const int lane = lane_id();
   const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
   int64_t x = 0, y = blockIdx.x;
@@ -470,6 +512,7 @@ struct FinArgs {
   const float* part;   // [cs][Np] row partials per column split
   const float* cpart;  // [Np][rb] column partials per row block
   int64_t tiles, col_tiles, rb, Np, N;
+  int32_t* flag;      // GramArgs
   float* r;           // workspace row sums
   float* s;           // workspace strengths (zero past N)
   float* out_s;       // optional outputs
@@ -478,33 +521,45 @@ struct FinArgs {
   float* out_f;
 };
 
+// Row i of block xi: its splits' row partials, then the column partials of
+// the blocks above it. FIN_LANES lanes per row, each summing a fixed strided
+// subset (a row's column partials are contiguous), added by a butterfly (one
+// lane per row: 9.7 against 4.7 us at 8192 positions).
+// Pass 0 writes T and F for weights that are all 1; pass 1 replaces them where
+// some are not (GramArgs::flag).
+constexpr int FIN_LANES = 8;
 template <int PASS>
 __global__ __launch_bounds__(256) void gram_finalize_kernel(FinArgs a) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (PASS == 1 && *a.flag == 0) return;
+  const int64_t i = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) / FIN_LANES;
+  const int sub = threadIdx.x % FIN_LANES;
   if (i >= a.Np) return;
-  // Row i of block xi: its splits' row partials, then the column partials
-  // of the blocks above it, in order.
   const int64_t xi = i / GRAM_ROWS;
   const int64_t ns = gram_splits(xi, a.tiles, a.col_tiles);
   float sum = 0.f;
-  for (int64_t c = 0; c < ns; ++c) sum += a.part[c * a.Np + i];
+  for (int64_t c = sub; c < ns; c += FIN_LANES) sum += a.part[c * a.Np + i];
   const float* cp = a.cpart + i * a.rb;
-  for (int64_t xb = 0; xb < xi; ++xb) sum += cp[xb];
+#pragma unroll 4
+  for (int64_t xb = sub; xb < xi; xb += FIN_LANES) sum += cp[xb];
+#pragma unroll
+  for (int off = FIN_LANES / 2; off >= 1; off >>= 1) sum += shfl_xor_f32(sum, off);
+  if (sub != 0) return;
+  float s;
   if constexpr (PASS == 0) {
-    const float s = i < a.N ? sum / (sum + 1e-8f) : 0.f;
+    s = i < a.N ? sum / (sum + 1e-8f) : 0.f;
     a.r[i] = sum;
     a.s[i] = s;
-    if (i < a.N) {
-      if (a.out_r) a.out_r[i] = sum;
-      if (a.out_s) a.out_s[i] = s;
-    }
+    if (i >= a.N) return;
+    if (!(s == 1.f)) *a.flag = 1;
+    if (a.out_r) a.out_r[i] = sum;
+    if (a.out_s) a.out_s[i] = s;
   } else {
     if (i >= a.N) return;
-    const float t = sum / (a.r[i] + 1e-8f);
-    const float s = a.s[i];
-    if (a.out_t) a.out_t[i] = t;
-    a.out_f[i] = 4.f * s - 2.f * s + 3.f * t;
+    s = a.s[i];
   }
+  const float t = sum / ((PASS == 0 ? sum : a.r[i]) + 1e-8f);
+  if (a.out_t) a.out_t[i] = t;
+  a.out_f[i] = 4.f * s - 2.f * s + 3.f * t;
 }
 
 template <typename T>
@@ -605,6 +660,7 @@ extern "C" cab_status_t cab_token_frc_from_keys(const void* keys, cab_dtype_t dt
   CAB_REQUIRE(valid_dtype(dtype), CAB_EDTYPE, "%s: unknown dtype %d", fn, static_cast<int>(dtype));
   CAB_REQUIRE(B >= 1 && H >= 1 && N >= 0 && D >= 1, CAB_ESHAPE, "%s: bad shape", fn);
   CAB_REQUIRE(D <= 256, CAB_ESHAPE, "%s: D %lld above 256", fn, static_cast<long long>(D));
+  CAB_REQUIRE(B <= INT32_MAX / H, CAB_ESHAPE, "%s: too many (batch, head) slices", fn);
   if (N == 0) return CAB_OK;
   CAB_REQUIRE(keys && frc && strides && workspace, CAB_EINVAL, "%s: null argument", fn);
   for (int d = 0; d < 4; ++d) CAB_REQUIRE(strides[d] >= 0, CAB_ESHAPE, "%s: negative stride", fn);
@@ -621,10 +677,11 @@ extern "C" cab_status_t cab_token_frc_from_keys(const void* keys, cab_dtype_t dt
   float* s = reinterpret_cast<float*>(ws + L.off_s);
   float* part = reinterpret_cast<float*>(ws + L.off_part);
   float* cpart = reinterpret_cast<float*>(ws + L.off_cpart);
+  int32_t* flag = reinterpret_cast<int32_t*>(ws + L.off_flag);
   hipStream_t st = static_cast<hipStream_t>(stream);
 
   PrepArgs pa{keys, H, B * H, N, D, L.Np, L.dk, {strides[0], strides[1], strides[2], strides[3]},
-              hi, lo};
+              hi, lo, flag};
   const unsigned pgrid = static_cast<unsigned>(L.Np / 4);
   // 16-byte loads when each position's D values are contiguous and every
   // row start (all b, h, n strides) keeps 16-byte alignment.
@@ -632,26 +689,27 @@ extern "C" cab_status_t cab_token_frc_from_keys(const void* keys, cab_dtype_t dt
   const bool vec = strides[3] == 1 && D % 8 == 0 && reinterpret_cast<uintptr_t>(keys) % 16 == 0 &&
                    (strides[0] * esz) % 16 == 0 && (strides[1] * esz) % 16 == 0 &&
                    (strides[2] * esz) % 16 == 0;
+  const auto prep = [&](auto t, auto v) {
+    using T = decltype(t);
+    constexpr bool VEC = decltype(v)::value;
+    if (L.dk == 4)
+      keys_prep_kernel<T, VEC, 8><<<pgrid, 256, 0, st>>>(pa);
+    else if (L.dk == 8)
+      keys_prep_kernel<T, VEC, 16><<<pgrid, 256, 0, st>>>(pa);
+    else
+      keys_prep_kernel<T, VEC, 32><<<pgrid, 256, 0, st>>>(pa);
+  };
   switch (dtype) {
-    case CAB_F32:
-      vec ? keys_prep_kernel<float, true><<<pgrid, 256, 0, st>>>(pa)
-          : keys_prep_kernel<float, false><<<pgrid, 256, 0, st>>>(pa);
-      break;
-    case CAB_BF16:
-      vec ? keys_prep_kernel<bf16_t, true><<<pgrid, 256, 0, st>>>(pa)
-          : keys_prep_kernel<bf16_t, false><<<pgrid, 256, 0, st>>>(pa);
-      break;
-    default:
-      vec ? keys_prep_kernel<f16_t, true><<<pgrid, 256, 0, st>>>(pa)
-          : keys_prep_kernel<f16_t, false><<<pgrid, 256, 0, st>>>(pa);
-      break;
+    case CAB_F32: vec ? prep(float{}, std::true_type{}) : prep(float{}, std::false_type{}); break;
+    case CAB_BF16: vec ? prep(bf16_t{}, std::true_type{}) : prep(bf16_t{}, std::false_type{}); break;
+    default: vec ? prep(f16_t{}, std::true_type{}) : prep(f16_t{}, std::false_type{}); break;
   }
   cab_status_t rc = launch_status(fn);
   if (rc != CAB_OK) return rc;
 
-  GramArgs g{hi, lo, s, part, cpart, L.Np, L.tiles, L.col_tiles, L.rb};
-  FinArgs f{part, cpart, L.tiles, L.col_tiles, L.rb, L.Np, N, r, s, strengths, triangles, row_sums, frc};
-  const unsigned fgrid = static_cast<unsigned>(ceil_div(L.Np, 256));
+  GramArgs g{hi, lo, s, part, cpart, flag, L.Np, L.tiles, L.col_tiles, L.rb};
+  FinArgs f{part, cpart, L.tiles, L.col_tiles, L.rb, L.Np, N, flag, r, s, strengths, triangles, row_sums, frc};
+  const unsigned fgrid = static_cast<unsigned>(ceil_div(L.Np * FIN_LANES, 256));
   for (int pass = 0; pass < 2; ++pass) {
     if (L.dk == 4) {
       pass == 0 ? launch_gram<4, 0>(g, L, st) : launch_gram<4, 1>(g, L, st);
