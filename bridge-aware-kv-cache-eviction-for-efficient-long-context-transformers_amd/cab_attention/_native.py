@@ -83,6 +83,10 @@ SIGNATURES = {
     "cab_evict_connectivity": (ctypes.c_int, [_ptr, _i64, _i64, _ptr, _ptr, _ptr]),
     "cab_kv_gather": (ctypes.c_int, [ctypes.POINTER(_ptr), ctypes.POINTER(_ptr), _i32, _i64, _i64,
                                      _i64, _i64, _i64x4, _i64x4, _ptr, _i64, _ptr]),
+    "cab_kv_append": (ctypes.c_int, [_ptr, _ptr, _ptr, _ptr, _i32, _i64, _i64, _i64, _i64, _i64x4,
+                                     _i64x4, _i64x4, _i64, _ptr]),
+    "cab_key_sums": (ctypes.c_int, [_ptr, ctypes.c_int, _i64, _i64, _i64, _i64, _i64x4, _ptr, _i64,
+                                    _ptr, _ptr]),
     "cab_token_frc": (ctypes.c_int, [_ptr, ctypes.c_int, _i64, _i64, _ptr, _ptr, _ptr, _ptr]),
     "cab_attention_symmetrize": (ctypes.c_int, [_ptr, ctypes.c_int, _i64, _i64, _i64, _i64, _i64x4,
                                                 _ptr, _i64, _ptr]),

@@ -18,6 +18,31 @@ def _rows_aligned(t: torch.Tensor) -> bool:
             and all((s * es) % 16 == 0 for s in t.stride()[:3]))
 
 
+_APPEND_DTYPES = (torch.bfloat16, torch.float16, torch.float32)
+
+
+def append_rows(k: torch.Tensor, v: torch.Tensor, k_dst: torch.Tensor, v_dst: torch.Tensor,
+                row: int) -> bool:
+    """Copies ``k``, ``v`` ``[B, H, n, D]`` to rows ``row ..`` of the buffers
+    ``[B, H, capacity, >= D]`` (one stride set, contiguous last dim) in one
+    launch (``cab_kv_append``). False, and nothing done, for what the kernel
+    does not take (another device or dtype, gradients to record)."""
+    dev = k_dst.device
+    if (dev.type != "cuda" or k.device != dev or v.device != dev
+            or k.dtype not in _APPEND_DTYPES or k_dst.dtype != k.dtype
+            or (torch.is_grad_enabled() and (k.requires_grad or v.requires_grad
+                                             or k_dst.requires_grad or v_dst.requires_grad))):
+        return False
+    B, H, n, D = k.shape
+    with torch.cuda.device(dev):
+        st = nat.load().cab_kv_append(k.data_ptr(), v.data_ptr(), k_dst.data_ptr(),
+                                      v_dst.data_ptr(), k.element_size(), B, H, n, D,
+                                      nat.strides4(k), nat.strides4(v), nat.strides4(k_dst), row,
+                                      nat.stream_ptr(dev))
+    nat.check("cab_kv_append", st)
+    return True
+
+
 def gather_into(srcs: Sequence[torch.Tensor], dsts: Sequence[torch.Tensor],
                 keep_indices: torch.Tensor, n_src: int, validate: bool = True) -> None:
     """``dst[:, :, t, :] = src[:, :, keep[t], :]`` for pairs of ``[B, H, *, D]``

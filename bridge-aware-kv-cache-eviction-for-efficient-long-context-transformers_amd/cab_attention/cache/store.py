@@ -32,7 +32,7 @@ from typing import Any, Callable, Dict, List, Optional, Tuple
 import torch
 
 from ..scoring import ImportanceTracker
-from .prune import gather_into
+from .prune import append_rows, gather_into
 
 _GRAIN = 16  # bytes: rows are padded to whole 16-byte chunks for the gather kernel
 
@@ -62,7 +62,8 @@ class LayeredKV:
 
     def _alloc(self, like: torch.Tensor, capacity: int, width: int) -> torch.Tensor:
         B, H = like.shape[0], like.shape[1]
-        return torch.zeros((B, H, capacity, width), dtype=like.dtype, device=like.device)
+        # (rows are written before they are read, padding columns never read)
+        return torch.empty((B, H, capacity, width), dtype=like.dtype, device=like.device)
 
     # -- rows -------------------------------------------------------------
     def length(self, layer: int) -> int:
@@ -100,8 +101,9 @@ class LayeredKV:
             nv[:, :, :L.length].copy_(L.v[:, :, :L.length])
             L.k, L.v = nk, nv
             L.k_spare = L.v_spare = None  # reallocated at the next prune
-        L.k[:, :, L.length:need, :L.width].copy_(k)
-        L.v[:, :, L.length:need, :L.width].copy_(v)
+        if not append_rows(k, v, L.k, L.v, L.length):
+            L.k[:, :, L.length:need, :L.width].copy_(k)
+            L.v[:, :, L.length:need, :L.width].copy_(v)
         L.length = need
 
     def capacity(self, layer: int) -> int:

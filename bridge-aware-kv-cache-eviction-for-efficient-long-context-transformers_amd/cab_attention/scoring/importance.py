@@ -1,6 +1,6 @@
 """Cumulative-attention (H2O) importance tracking (reference:
 ``cab_attention/scoring/importance.py`` :17-133). The running totals are
-torch bookkeeping; the top-k runs in ``cab_evict_select``."""
+summed by ``cab_key_sums`` on the GPU; the top-k runs in ``cab_evict_select``."""
 
 from __future__ import annotations
 
@@ -8,7 +8,10 @@ from typing import Optional
 
 import torch
 
+from .. import _native as nat
 from ..eviction._select import BRIDGE_NONE, select_positions
+
+_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
 
 
 class ImportanceTracker:
@@ -26,6 +29,8 @@ class ImportanceTracker:
     def update(self, attention_weights: torch.Tensor):
         """Adds ``attention_weights [B, H, N_q, N_kv]`` summed over batch,
         heads and queries; a longer N_kv extends the totals with zeros."""
+        if self._update_on_device(attention_weights):
+            return
         position_scores = attention_weights.sum(dim=(0, 1, 2)).float()
         if self.cumulative_scores is None:
             self.cumulative_scores = position_scores
@@ -38,6 +43,32 @@ class ImportanceTracker:
                                 dtype=self.cumulative_scores.dtype)])
             self.cumulative_scores[:cur] += position_scores
         self.total_queries += attention_weights.shape[2]
+
+    def _update_on_device(self, w: torch.Tensor) -> bool:
+        """:meth:`update` in one launch (``cab_key_sums``), the extension
+        included. False, and nothing done, for what it does not take."""
+        old = self.cumulative_scores
+        if (w.device.type != "cuda" or w.dim() != 4 or w.dtype not in _DTYPES or w.numel() == 0
+                or (w.requires_grad and torch.is_grad_enabled())):
+            return False
+        B, H, n_q, n_k = w.shape
+        if old is None:
+            n_old = 0
+        elif (old.device != w.device or old.dtype != torch.float32 or old.dim() != 1
+              or not old.is_contiguous() or old.requires_grad):
+            return False
+        else:
+            n_old = old.numel()
+        # Totals that reach far enough are added to in place, shorter ones extended.
+        sums = old if n_old >= n_k else torch.empty(n_k, dtype=torch.float32, device=w.device)
+        with torch.cuda.device(w.device):
+            st = nat.load().cab_key_sums(w.data_ptr(), nat.dtype_code(w), B, H, n_q, n_k,
+                                         nat.strides4(w), nat.ptr(old), n_old, sums.data_ptr(),
+                                         nat.stream_ptr(w.device))
+        nat.check("cab_key_sums", st)
+        self.cumulative_scores = sums
+        self.total_queries += n_q
+        return True
 
     def add_scores(self, position_scores: torch.Tensor, n_queries: int = 1):
         """Adds per-position totals already summed over queries (for example

@@ -403,6 +403,30 @@ cab_status_t cab_kv_gather(const void* const* src, void* const* dst, int32_t n_t
                            const int64_t* keep_indices, int64_t n_keep, void* stream);
 
 /*
+ * The caches' per-step work (CABCache.update, cache/cab_cache.py:122-175):
+ *
+ * cab_kv_append copies new K and V rows [B,H,n,D] (element strides; elements
+ * of element_bytes = 2 or 4) behind the rows a layer holds: rows dst_row ..
+ * dst_row + n - 1 of k_dst and v_dst, two buffers of one stride set
+ * {b, h, row, 1}. One launch for both.
+ *
+ * cab_key_sums replaces the sum of ImportanceTracker.update
+ * (scoring/importance.py:35-70): sums[j] = (j < n_old ? old_sums[j] : 0) +
+ * sum over b, h, q of attention[b,h,q,j], j < N_k, summed in fp32 in a fixed
+ * order; of 16-bit weights the sum is rounded to their type before it is
+ * added. old_sums may be sums itself.
+ */
+cab_status_t cab_kv_append(const void* k, const void* v, void* k_dst, void* v_dst,
+                           int32_t element_bytes, int64_t B, int64_t H, int64_t n, int64_t D,
+                           const int64_t k_strides[4], const int64_t v_strides[4],
+                           const int64_t dst_strides[4], int64_t dst_row, void* stream);
+
+cab_status_t cab_key_sums(const void* attention, cab_dtype_t dtype, int64_t B, int64_t H,
+                          int64_t N_q, int64_t N_k, const int64_t strides[4],
+                          const float* old_sums, int64_t n_old, float* sums, void* stream);
+
+
+/*
  * Token-level Forman-Ricci curvature of a weighted directed graph A [n, n]
  * (compute_frc / compute_frc_triton / compute_frc_pytorch,
  * cab_attention/kernels/frc_triton.py:21-314):

@@ -1,0 +1,104 @@
+"""cab_kv_append and cab_key_sums: the appended rows bit for bit whatever the
+strides, alignment and element size, and the sums against torch in float64."""
+
+import ctypes
+
+import pytest
+import torch
+
+from cab_attention import _native as nat
+
+gpu = pytest.mark.gpu
+
+
+@gpu
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,H,n,D,layout", [
+    (1, 8, 1, 128, "plain"),        # a decode step: 16-byte units
+    (2, 3, 300, 64, "plain"),
+    (1, 2, 5, 20, "plain"),         # rows of no whole 16 bytes (bf16), padded buffer
+    (2, 4, 33, 128, "transposed"),  # [B, n, H, D] as a projection leaves it
+    (1, 2, 7, 64, "strided"),       # last-dim stride 2
+    (1, 2, 9, 64, "offset"),        # rows one element past a 16-byte boundary
+    (1, 1, 1, 1, "plain"),
+])
+def test_append_matches_copy(cuda, dt, B, H, n, D, layout):
+    from cab_attention.cache.store import LayeredKV
+    g = torch.Generator().manual_seed(n + D)
+
+    def make():
+        if layout == "transposed":
+            return torch.randn((B, n, H, D), generator=g).to(dt).to(cuda).transpose(1, 2)
+        if layout == "strided":
+            return torch.randn((B, H, n, 2 * D), generator=g).to(dt).to(cuda)[..., ::2]
+        if layout == "offset":
+            flat = torch.randn(B * H * n * D + 1, generator=g).to(dt).to(cuda)
+            return flat[1:].view(B, H, n, D)
+        return torch.randn((B, H, n, D), generator=g).to(dt).to(cuda)
+
+    store, want_k, want_v = LayeredKV(initial_capacity=4), [], []
+    for _ in range(3):  # the later ones grow the buffers
+        k, v = make(), make().contiguous()  # (K and V strides differ)
+        store.append(0, k, v)
+        want_k.append(k)
+        want_v.append(v)
+    got_k, got_v = store.view(0)
+    assert torch.equal(got_k, torch.cat(want_k, 2)) and torch.equal(got_v, torch.cat(want_v, 2))
+
+
+@gpu
+def test_append_keeps_gradients_to_torch(cuda):
+    from cab_attention.cache.store import LayeredKV
+    store = LayeredKV()
+    k = torch.randn((1, 2, 3, 64), device=cuda, requires_grad=True)
+    store.append(0, k, k.detach())
+    store.view(0)[0].sum().backward()
+    assert torch.equal(k.grad, torch.ones_like(k))
+
+
+@gpu
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,Nq,Nk,n_old", [(1, 32, 1, 2000, 1999), (1, 32, 16, 4500, 0),
+                                             (2, 3, 7, 63, 63), (1, 1, 1, 1, 0), (2, 8, 9, 65, 200)])
+def test_importance_update(cuda, dt, B, H, Nq, Nk, n_old):
+    from cab_attention.scoring import ImportanceTracker
+    g = torch.Generator(device=cuda).manual_seed(Nk)
+    full = torch.softmax(torch.randn((B, H, Nq, Nk + 3), generator=g, device=cuda), -1).to(dt)
+    w = full[..., :Nk]  # rows of a longer buffer
+    t = ImportanceTracker(device="cuda")
+    base = torch.zeros(max(n_old, Nk), dtype=torch.float64, device=cuda)
+    if n_old:
+        t.cumulative_scores = torch.rand(n_old, generator=g, device=cuda)
+        base[:n_old] = t.cumulative_scores.double()
+    before = t.cumulative_scores
+    t.update(w)
+    got = t.get_scores()
+    assert (got is before) == (n_old >= Nk) and t.total_queries == Nq
+    base[:Nk] += w.double().sum((0, 1, 2))
+    # fp32 sums of non-negative terms; 16-bit sums end rounded to their type
+    ulp = {torch.float32: 2e-6, torch.bfloat16: 2 ** -8, torch.float16: 2 ** -11}[dt]
+    torch.testing.assert_close(got.double(), base, rtol=ulp, atol=1e-7)
+
+
+def test_cache_ops_validation():
+    lib = nat.load()
+    s = (ctypes.c_int64 * 4)(64, 64, 64, 1)
+    bad = (ctypes.c_int64 * 4)(64, 64, 64, 2)
+    fake = 0x7f0000000000
+    app = lambda **kw: lib.cab_kv_append(  # noqa: E731
+        kw.get("k", fake), fake, kw.get("kd", fake), fake, kw.get("es", 2), kw.get("B", 1), 1,
+        kw.get("n", 1), 64, s, s, kw.get("ds", s), kw.get("row", 0), None)
+    assert app(es=8) == nat.CAB_EDTYPE
+    assert app(n=-1) == nat.CAB_ESHAPE and app(row=-1) == nat.CAB_ESHAPE
+    assert app(k=None) == nat.CAB_EINVAL
+    assert app(ds=bad) == nat.CAB_ESHAPE
+    assert app(k=fake + 1) == nat.CAB_ESHAPE
+    assert app(B=1 << 40) == nat.CAB_ESHAPE
+    assert app(n=0) == nat.CAB_OK
+    sums = lambda **kw: lib.cab_key_sums(  # noqa: E731
+        kw.get("a", fake), kw.get("dt", nat.CAB_F32), 1, 1, kw.get("Nq", 1), 64, s,
+        kw.get("old", None), kw.get("n_old", 0), fake, None)
+    assert sums(dt=9) == nat.CAB_EDTYPE
+    assert sums(Nq=0) == nat.CAB_ESHAPE
+    assert sums(a=None) == nat.CAB_EINVAL
+    assert sums(n_old=3) == nat.CAB_EINVAL
