@@ -7,6 +7,7 @@ CPU tensor or an ABI error raises.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 import pathlib
@@ -140,14 +141,14 @@ def check(fn: str, status: int) -> None:
         raise CabError(fn, status, msg)
 
 
+_DTYPE_CODES = {torch.float32: CAB_F32, torch.float16: CAB_F16, torch.bfloat16: CAB_BF16}
+
+
 def dtype_code(t: torch.Tensor) -> int:
-    if t.dtype == torch.float32:
-        return CAB_F32
-    if t.dtype == torch.float16:
-        return CAB_F16
-    if t.dtype == torch.bfloat16:
-        return CAB_BF16
-    raise TypeError(f"unsupported dtype {t.dtype}; expected float32, float16 or bfloat16")
+    code = _DTYPE_CODES.get(t.dtype)
+    if code is None:
+        raise TypeError(f"unsupported dtype {t.dtype}; expected float32, float16 or bfloat16")
+    return code
 
 
 def require_device(*tensors: torch.Tensor) -> torch.device:
@@ -155,7 +156,7 @@ def require_device(*tensors: torch.Tensor) -> torch.device:
     for t in tensors:
         if not isinstance(t, torch.Tensor):
             raise TypeError(f"expected a torch.Tensor, got {type(t).__name__}")
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise RuntimeError(
                 "CAB-Attention kernels run on the GPU only (HIP, gfx950); got a tensor on "
                 f"{t.device}. Move inputs to a cuda device.")
@@ -166,26 +167,47 @@ def require_device(*tensors: torch.Tensor) -> torch.device:
     return dev
 
 
+_I64x4 = ctypes.c_int64 * 4
+
+
 def strides4(t: torch.Tensor):
-    arr = (ctypes.c_int64 * 4)(*t.stride())
-    return arr
+    return _I64x4(*t.stride())
+
+
+def rows_aligned(t: torch.Tensor) -> bool:
+    """Last dim contiguous and rows starting on 16-byte boundaries (what the
+    kernels' vector loads need)."""
+    st = t.stride()
+    if st[-1] != 1 or t.data_ptr() & 15:
+        return False
+    bits = 0
+    for s in st[:-1]:
+        bits |= s
+    return (bits * t.element_size()) & 15 == 0
 
 
 def aligned_rows(t: torch.Tensor) -> torch.Tensor:
-    """Return ``t`` or a contiguous copy so that its last dim is contiguous and
-    rows start on 16-byte boundaries (what the kernels' vector loads need)."""
-    def ok(x):
-        es = x.element_size()
-        return (x.stride(-1) == 1 and x.data_ptr() % 16 == 0
-                and all((s * es) % 16 == 0 for s in x.stride()[:-1]))
-    if ok(t):
+    """Return ``t`` or a contiguous copy with :func:`rows_aligned` rows."""
+    if rows_aligned(t):
         return t
     t = t.contiguous()
-    return t if ok(t) else t.clone()
+    return t if rows_aligned(t) else t.clone()
+
+
+_SAME_DEVICE = contextlib.nullcontext()
+
+
+def on_device(device: torch.device):
+    """Context in which ``device`` is current (nothing to switch if it already
+    is, the usual case: a decode step's launches cost as much as their kernels)."""
+    if device.index is None or device.index == torch.cuda.current_device():
+        return _SAME_DEVICE
+    return torch.cuda.device(device)
 
 
 def stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    index = torch.cuda.current_device() if device.index is None else device.index
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def ptr(t):

@@ -13,9 +13,7 @@ import torch
 from .. import _native as nat
 
 def _rows_aligned(t: torch.Tensor) -> bool:
-    es = t.element_size()
-    return (t.stride(3) == 1 and t.data_ptr() % 16 == 0 and (t.shape[3] * es) % 16 == 0
-            and all((s * es) % 16 == 0 for s in t.stride()[:3]))
+    return nat.rows_aligned(t) and (t.shape[3] * t.element_size()) % 16 == 0
 
 
 _APPEND_DTYPES = (torch.bfloat16, torch.float16, torch.float32)
@@ -34,7 +32,7 @@ def append_rows(k: torch.Tensor, v: torch.Tensor, k_dst: torch.Tensor, v_dst: to
                                              or k_dst.requires_grad or v_dst.requires_grad))):
         return False
     B, H, n, D = k.shape
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         st = nat.load().cab_kv_append(k.data_ptr(), v.data_ptr(), k_dst.data_ptr(),
                                       v_dst.data_ptr(), k.element_size(), B, H, n, D,
                                       nat.strides4(k), nat.strides4(v), nat.strides4(k_dst), row,
@@ -74,7 +72,7 @@ def gather_into(srcs: Sequence[torch.Tensor], dsts: Sequence[torch.Tensor],
     lib = nat.load()
     src_arr = (ctypes.c_void_p * len(srcs))(*[s.data_ptr() for s in srcs])
     dst_arr = (ctypes.c_void_p * len(dsts))(*[d.data_ptr() for d in dsts])
-    with torch.cuda.device(dev):  # the library launches one kernel per 32 tensors
+    with nat.on_device(dev):  # the library launches one kernel per 32 tensors
         st = lib.cab_kv_gather(src_arr, dst_arr, len(srcs), B, H, n_src, D * es, ss, ds,
                                keep_indices.data_ptr(), n_keep, nat.stream_ptr(dev))
     nat.check("cab_kv_gather", st)

@@ -75,7 +75,10 @@ class LayeredKV:
         if layer >= len(self.layers) or self.layers[layer] is None:
             return None, None
         L = self.layers[layer]
-        return L.k[:, :, :L.length, :L.width], L.v[:, :, :L.length, :L.width]
+        k, v = L.k.narrow(2, 0, L.length), L.v.narrow(2, 0, L.length)
+        if L.width != L.k.shape[3]:
+            k, v = k.narrow(3, 0, L.width), v.narrow(3, 0, L.width)
+        return k, v
 
     def append(self, layer: int, k: torch.Tensor, v: torch.Tensor):
         if k.dim() != 4 or v.shape != k.shape or v.dtype != k.dtype:

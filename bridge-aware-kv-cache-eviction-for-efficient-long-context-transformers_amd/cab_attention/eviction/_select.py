@@ -56,7 +56,7 @@ def select_positions(cache_len: int, scores: torch.Tensor | None, local: int, im
     # Large caches run one workgroup per segment with a workspace.
     wbytes = int(lib.cab_evict_select_workspace_bytes(cache_len)) if cache_len >= MULTI_MIN else 0
     ws = torch.empty(wbytes, dtype=torch.uint8, device=dev) if wbytes else None
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         st = lib.cab_evict_select(nat.ptr(scores), 0 if scores is None else scores.numel(),
                                   nat.ptr(bridge_scores), cache_len, local, imp, bridge,
                                   int(bool(fallback)), mode, keep.data_ptr(), counts.data_ptr(),
@@ -80,7 +80,7 @@ def connectivity(attention: torch.Tensor, category: torch.Tensor) -> torch.Tenso
         a = a.contiguous()
     out = torch.empty(max(n, 1), dtype=torch.float32, device=dev)
     lib = nat.load()
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         st = lib.cab_evict_connectivity(a.data_ptr(), n, a.stride(0), category.data_ptr(),
                                         out.data_ptr(), nat.stream_ptr(dev))
     nat.check("cab_evict_connectivity", st)

@@ -47,7 +47,7 @@ def coarsen_qk_max_l2(q: torch.Tensor, k: torch.Tensor, block_size: int = 64,
     kc = torch.empty((B, H, M, D), dtype=k.dtype, device=dev)
     qi = torch.empty((B, H, M), dtype=torch.int32, device=dev) if return_indices else None
     ki = torch.empty((B, H, M), dtype=torch.int32, device=dev) if return_indices else None
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         st = lib.cab_coarsen_maxl2(q.data_ptr(), k.data_ptr(), dt, B, H, N, D,
                                    nat.strides4(q), nat.strides4(k), block_size,
                                    qc.data_ptr(), kc.data_ptr(), nat.ptr(qi), nat.ptr(ki),

@@ -86,7 +86,7 @@ def _dense(q, k, v, scale, causal, out=None, want_lse=False, old=None, scores=No
     wbytes = lib.cab_flash_attn_scores_workspace_bytes(dt, B, H, H_kv, N_q, N_k, D, ks, vs,
                                                        int(scores is not None))
     ws = torch.empty(max(int(wbytes), 16), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         st = lib.cab_flash_attn_scores_fwd(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), dt, B, H, H_kv, N_q, N_k, D,
             nat.strides4(q), ks, vs, nat.strides4(out), float(scale), int(bool(causal)),
@@ -125,7 +125,7 @@ def key_scores(q: torch.Tensor, k: torch.Tensor, lse: torch.Tensor, scale: float
     if scale is None:
         scale = 1.0 / math.sqrt(D)
     st3 = nat.strides4(scores)  # [b, h, token] strides (the 4th slot is unused)
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         st = lib.cab_attn_key_scores(q.data_ptr(), k.data_ptr(), lse.data_ptr(), dt, B, H, H_kv,
                                      N_q, N_k, D, nat.strides4(q), nat.strides4(k), float(scale),
                                      int(bool(causal)), scores.data_ptr(), st3,

@@ -68,7 +68,7 @@ def compute_block_frc(q_coarse: torch.Tensor, k_coarse: torch.Tensor, temperatur
     form = nat.FORMULAS[formula]
     wbytes = lib.cab_block_frc_workspace_bytes(B, H, M, D, norm, form)
     ws = torch.empty(max(int(wbytes), 1), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         st = lib.cab_block_frc(qc.data_ptr(), kc.data_ptr(), dt, B, H, M, D,
                                1.0 / math.sqrt(D), float(temperature), float(lambda_redundancy),
                                norm, form, frc.data_ptr(), nat.ptr(aff), nat.ptr(tri),
@@ -104,7 +104,7 @@ def _select(frc: torch.Tensor, sparsity: float, select_high: bool, keep_diagonal
     kv_cnt = torch.empty((B, H, M), dtype=torch.int32, device=dev)
     mask = torch.empty((B, H, M, M), dtype=torch.bool, device=dev) if dense else None
     flags = (int(bool(select_high)), int(bool(keep_diagonal)), int(bool(causal)))
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         if magnitude_scores is None:
             name = "cab_block_topk"
             st = lib.cab_block_topk(f.data_ptr(), B, H, M, k, *flags, kv_idx.data_ptr(),

@@ -80,7 +80,7 @@ def block_sparse_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     wbytes = lib.cab_block_sparse_attn_workspace_bytes_k(dt, B, H, N, D, int(block_size),
                                                          int(kv_idx.shape[-1]))
     ws = torch.empty(max(int(wbytes), 16), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         st = lib.cab_block_sparse_attn_fwd(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), dt, B, H, N, D, nat.strides4(q),
             nat.strides4(k), nat.strides4(v), nat.strides4(out), int(block_size),
@@ -104,7 +104,7 @@ def pack_v(v: torch.Tensor, block_size: int = 64) -> torch.Tensor:
     v = nat.aligned_rows(v)
     wbytes = lib.cab_block_sparse_attn_workspace_bytes(dt, B, H, N, D, int(block_size))
     vt = torch.empty(max(int(wbytes), 16), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         st = lib.cab_block_sparse_attn_pack_v(v.data_ptr(), dt, B, H, N, D, nat.strides4(v),
                                               int(block_size), vt.data_ptr(), vt.numel(),
                                               nat.stream_ptr(dev))
@@ -136,7 +136,7 @@ def block_sparse_attention_packed(q: torch.Tensor, k: torch.Tensor, vt: torch.Te
     out, lse = _outputs(q, out, return_lse, dev)
     if scale is None:
         scale = 1.0 / math.sqrt(D)
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         st = lib.cab_block_sparse_attn_fwd_packed(
             q.data_ptr(), k.data_ptr(), vt.data_ptr(), dt, B, H, N, D, nat.strides4(q),
             nat.strides4(k), nat.strides4(out), int(block_size), kv_idx.data_ptr(),

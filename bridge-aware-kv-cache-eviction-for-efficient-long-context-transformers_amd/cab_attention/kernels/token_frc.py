@@ -37,7 +37,7 @@ def token_frc(attention: torch.Tensor, return_parts: bool = False):
     t = torch.empty(n, dtype=torch.float32, device=dev)
     f = torch.empty(n, dtype=torch.float32, device=dev)
     lib = nat.load()
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         st = lib.cab_token_frc(a.data_ptr(), dt, n, a.stride(0) if n else 0, s.data_ptr(),
                                t.data_ptr(), f.data_ptr(), nat.stream_ptr(dev))
     nat.check("cab_token_frc", st)
@@ -86,7 +86,7 @@ def symmetrize_attention(attention: torch.Tensor) -> torch.Tensor:
     n = max(nq, nk)
     out = torch.empty((n, n), dtype=torch.float32, device=dev)
     lib = nat.load()
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         st = lib.cab_attention_symmetrize(attention.data_ptr(), dt, B, H, nq, nk,
                                           nat.strides4(attention), out.data_ptr(), n,
                                           nat.stream_ptr(dev))
@@ -118,7 +118,7 @@ def frc_from_keys(keys: torch.Tensor, return_parts: bool = False):
         return ({**parts, "frc": f} if return_parts else f)
     wbytes = int(lib.cab_token_frc_keys_workspace_bytes(N, D))
     ws = torch.empty(wbytes, dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         st = lib.cab_token_frc_from_keys(
             keys.data_ptr(), dt, B, H, N, D, nat.strides4(keys),
             nat.ptr(parts and parts["strengths"]), nat.ptr(parts and parts["triangles"]),

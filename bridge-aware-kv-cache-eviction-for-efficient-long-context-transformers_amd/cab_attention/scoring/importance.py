@@ -61,7 +61,7 @@ class ImportanceTracker:
             n_old = old.numel()
         # Totals that reach far enough are added to in place, shorter ones extended.
         sums = old if n_old >= n_k else torch.empty(n_k, dtype=torch.float32, device=w.device)
-        with torch.cuda.device(w.device):
+        with nat.on_device(w.device):
             st = nat.load().cab_key_sums(w.data_ptr(), nat.dtype_code(w), B, H, n_q, n_k,
                                          nat.strides4(w), nat.ptr(old), n_old, sums.data_ptr(),
                                          nat.stream_ptr(w.device))
