@@ -1255,6 +1255,146 @@ __global__ __launch_bounds__(WI * WJ * 64, 1) void triangle_kernel(TriArgs a) {
     epilogue(std::integral_constant<int, CAB_FRC_AUGMENTED>{});
 }
 
+// ---------------------------------------------------------------------------
+// frc_small_kernel: the whole of cab_block_frc for M <= 128 under minmax
+// normalisation with the additive or multiplicative formula (the predictor's
+// prompts up to 8192 tokens at block size 64), one workgroup of 16 waves per
+// (b, h). Wave w owns the 32 x 32 tile (w / 4, w % 4) of A, of Ahat and of T alike:
+//   A = alpha Qc Kc^T, operands straight from global memory;
+//   min / max through LDS;
+//   Ahat stays in registers in fp32, X = f16(Ahat) goes to LDS row-major and
+//   transposed (the two MFMA operands; zero past M);
+//   T = X X with fp32 accumulate, and F from Ahat and T in registers.
+// Against STATS, EMIT, (min / max) and the triangle kernel this saves two or
+// three launches and the planes' round trip; launch and load latency bound it.
+// cab_block_frc, (b, h) x M x D, general path -> here: 8 x 16 x 128 fp16 18.9 -> 5.8
+// us, 8 x 128 x 128 bf16 17.8 -> 15.1, 512 x 128 x 128 bf16 43.5 -> 33.6, 16 x 64 x 64
+// fp32 42.8 -> 8.7, 32 x 128 x 128 fp32 with diagnostics 84.5 -> 22.9.
+// Numerics as on the large path: one fp16 product per site for T; Ahat in F at
+// fp32 accuracy (the fused additive form rounds it to fp16).
+// ---------------------------------------------------------------------------
+constexpr int SMALL_M = 128;
+
+struct SmallArgs {
+  const void* qc;
+  const void* kc;
+  int32_t M, D, formula;
+  float alpha, lambda;
+  float* frc;
+  float* affinity;   // or null
+  float* triangles;  // or null
+};
+
+template <typename T>
+__global__ __launch_bounds__(1024) void frc_small_kernel(SmallArgs a) {
+  constexpr int LD = SMALL_M + 8;  // 16-byte rows, spread over the banks
+  __shared__ __attribute__((aligned(16))) uint16_t xs[SMALL_M][LD], xt[SMALL_M][LD];
+  __shared__ float red[2][16];
+  const int w = threadIdx.x >> 6, lane = lane_id(), half = lane >> 5, l32 = lane & 31;
+  const int row0 = 32 * (w >> 2), col0 = 32 * (w & 3);
+  const int M = a.M, D = a.D;
+  const bool live = row0 < M && col0 < M;  // (uniform) a tile with elements
+  const size_t off = static_cast<size_t>(blockIdx.x) * M * D * sizeof(T);
+  const char* qb = static_cast<const char*>(a.qc) + off;
+  const char* kb = static_cast<const char*>(a.kc) + off;
+
+  f32x16 acc = {};
+  if (live) {
+    const int qr = row0 + l32, kr = col0 + l32;
+    const bool qin = qr < M, kin = kr < M;
+    if constexpr (sizeof(T) == 4) {
+      const float* q = reinterpret_cast<const float*>(qb) + static_cast<size_t>(qin ? qr : 0) * D;
+      const float* k = reinterpret_cast<const float*>(kb) + static_cast<size_t>(kin ? kr : 0) * D;
+#pragma unroll 4
+      for (int k0 = 0; k0 < D; k0 += 8) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(q + k0 + 4 * half);
+        const f32x4 y = *reinterpret_cast<const f32x4*>(k + k0 + 4 * half);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], y[e], acc, 0, 0, 0);
+      }
+    } else {
+      const uint16_t* q = reinterpret_cast<const uint16_t*>(qb) + static_cast<size_t>(qin ? qr : 0) * D;
+      const uint16_t* k = reinterpret_cast<const uint16_t*>(kb) + static_cast<size_t>(kin ? kr : 0) * D;
+#pragma unroll 8
+      for (int k0 = 0; k0 < D; k0 += 16) {
+        const bool in = k0 + 8 * half < D;  // D % 16 == 8: the upper half is past the row
+        const u32x4 x = in ? *reinterpret_cast<const u32x4*>(q + k0 + 8 * half) : u32x4{};
+        const u32x4 y = in ? *reinterpret_cast<const u32x4*>(k + k0 + 8 * half) : u32x4{};
+        if constexpr (std::is_same<T, bf16_t>::value)
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, x),
+                                                        __builtin_bit_cast(bf16x8, y), acc, 0, 0, 0);
+        else
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, x),
+                                                       __builtin_bit_cast(f16x8, y), acc, 0, 0, 0);
+      }
+    }
+  }
+  // Element e of the tile: row i0 + row_of(e), column j. (Rows and columns past
+  // M hold products of row 0 and are dropped here.)
+  const int i0 = row0 + 4 * half, j = col0 + l32;
+  auto row_of = [](int e) { return 8 * (e >> 2) + (e & 3); };
+  float mn = INFINITY, mx = -INFINITY;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+#pragma clang fp contract(off)
+    acc[e] = acc[e] * a.alpha;  // rounded by itself: the minimum maps to exactly 0
+    const bool in = i0 + row_of(e) < M && j < M;
+    mn = fminf(mn, in ? acc[e] : INFINITY);
+    mx = fmaxf(mx, in ? acc[e] : -INFINITY);
+  }
+#pragma unroll
+  for (int s = 1; s < 64; s <<= 1) {
+    mn = fminf(mn, shfl_xor_f32(mn, s));
+    mx = fmaxf(mx, shfl_xor_f32(mx, s));
+  }
+  if (lane == 0) {
+    red[0][w] = mn;
+    red[1][w] = mx;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    mn = fminf(mn, red[0][q]);
+    mx = fmaxf(mx, red[1][q]);
+  }
+  // A constant A stays as it is (outside fp16's range, perhaps): T = M c^2 below.
+  const bool constant = !(mx > mn);
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const bool in = i0 + row_of(e) < M && j < M;
+    acc[e] = in ? normalize_minmax(acc[e], mn, mx) : 0.f;
+    xs[i0 + row_of(e)][j] = constant ? uint16_t{0} : f32_to_f16(acc[e]);
+  }
+#pragma unroll
+  for (int e = 0; e < 16; e += 4) {
+    uint16_t h[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) h[q] = constant ? uint16_t{0} : f32_to_f16(acc[e + q]);
+    *reinterpret_cast<u32x2*>(&xt[j][i0 + row_of(e)]) =
+        u32x2{h[0] | static_cast<uint32_t>(h[1]) << 16, h[2] | static_cast<uint32_t>(h[3]) << 16};
+  }
+  __syncthreads();
+  if (!live) return;
+  f32x16 t = {};
+  for (int k0 = 0; k0 < M; k0 += 16)
+    t = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+        __builtin_bit_cast(f16x8, *reinterpret_cast<const u32x4*>(&xs[row0 + l32][k0 + 8 * half])),
+        __builtin_bit_cast(f16x8, *reinterpret_cast<const u32x4*>(&xt[col0 + l32][k0 + 8 * half])), t,
+        0, 0, 0);
+  if (j >= M) return;
+  const size_t base = static_cast<size_t>(blockIdx.x) * M * M + static_cast<size_t>(i0) * M + j;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const int r = row_of(e);
+    if (i0 + r >= M) continue;
+    const float tv = constant ? static_cast<float>(M) * acc[e] * acc[e] : t[e];
+    a.frc[base + r * M] = frc_combine(a.formula, acc[e], tv, a.lambda, 0.f, 0.f);
+    if (a.affinity) a.affinity[base + r * M] = acc[e];
+    if (a.triangles) a.triangles[base + r * M] = tv;
+  }
+}
+
 // Compute units of the current device (queried once per device).
 int device_cus() {
   static std::atomic<int> cached[64];
@@ -1386,6 +1526,18 @@ extern "C" cab_status_t cab_block_frc(const void* qc, const void* kc, cab_dtype_
   a.fused = fused ? 1 : 0;
   a.lambda = lambda_redundancy;
   a.strip = 1;
+
+  if (f16 && M <= SMALL_M) {
+    const SmallArgs sa{qc, kc, static_cast<int32_t>(M), static_cast<int32_t>(D), formula, a.alpha,
+                       lambda_redundancy, frc, affinity, triangles};
+    const unsigned grid = static_cast<unsigned>(BH);
+    switch (dtype) {
+      case CAB_BF16: frc_small_kernel<bf16_t><<<grid, 1024, 0, s>>>(sa); break;
+      case CAB_F16: frc_small_kernel<f16_t><<<grid, 1024, 0, s>>>(sa); break;
+      default: frc_small_kernel<float><<<grid, 1024, 0, s>>>(sa); break;
+    }
+    return launch_status("cab_block_frc/small");
+  }
 
   a.nparts = 0;
   if (normalization == CAB_NORM_MINMAX) {
