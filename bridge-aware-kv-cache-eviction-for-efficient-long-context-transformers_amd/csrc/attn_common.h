@@ -75,6 +75,15 @@ __device__ __forceinline__ void colmax2(float& x0, float& x1) {
   x1 = __builtin_bit_cast(float, b);
 }
 
+// Transposing LDS read (gfx950 ds_read_b64_tr_b16): the 16 lanes of a group
+// pass the addresses of a 4 x 16 block of 16-bit values, lane i the four at
+// row i / 4, columns 4 (i % 4) ..; lane i gets column i, rows 0 .. 3.
+__device__ __forceinline__ u32x2 lds_read_tr16(const void* p) {
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p));
+}
+
 // Running-max sentinel: a finite stand-in for -inf, so that -max * c stays
 // finite and exp2(s * c - max * c) of a masked score (-inf) is exactly 0.
 constexpr float M_EMPTY = -1.0e30f;

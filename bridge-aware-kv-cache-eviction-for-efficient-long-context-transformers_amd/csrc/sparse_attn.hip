@@ -92,7 +92,8 @@ struct AttnArgs {
   const uint16_t* vt;  // per (b, h, key block): V^T tile (16 KB) or fp32 block image (64 KB)
   void* o;             // same dtype as q
   float* lse;
-  int64_t qs[3], ks[3], os[3];  // b, h, token strides (elements)
+  const uint16_t* v;   // attn_pair_kernel with VROW: V's rows (vt unused)
+  int64_t qs[3], ks[3], os[3], vs[3];  // b, h, token strides (elements)
   const int32_t* kv_idx;
   const int32_t* kv_cnt;
   int32_t BH, H, N, M;  // B * H, query heads, query tokens, query blocks (all < 2^31)
@@ -972,7 +973,10 @@ __device__ __forceinline__ void pair_softmax(PairAcc<HD>& s, int r, f32x4 (&sc)[
   }
 }
 
-template <cab_dtype_t DT, int LIST, int HD>
+// VROW: V is staged as its rows, in K's LDS layout, and the V^T operands come
+// from transposing LDS reads; otherwise from packed V^T tiles (cab_..._packed).
+// ---------------------------------------------------------------------------
+template <cab_dtype_t DT, int LIST, int HD, bool VROW>
 __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
   static_assert(DT != CAB_F32, "16-bit inputs only");
   static_assert(LIST != LIST_GLOBAL, "lists staged in LDS, or dense");
@@ -1012,7 +1016,8 @@ __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
 
   const uint16_t* qb = static_cast<const uint16_t*>(a.q) + b * a.qs[0] + hh * a.qs[1];
   const char* kbytes = reinterpret_cast<const char*>(a.k + b * a.ks[0] + hk * a.ks[1]);
-  const char* vtbytes = reinterpret_cast<const char*>(a.vt) + bhk * Mk * TILE_BYTES;
+  const char* vtbytes = VROW ? reinterpret_cast<const char*>(a.v + b * a.vs[0] + hk * a.vs[1])
+                             : reinterpret_cast<const char*>(a.vt) + bhk * Mk * TILE_BYTES;
 
   // Queries (issued first; they land while the walk is built).
   PairAcc<HD> st;
@@ -1114,10 +1119,16 @@ __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
   // of the V^T tile of a block, one 1 KB buffer load each.
   const int64_t krow_bytes = a.ks[2] * 2;
   const int64_t kblk_bytes = BS * krow_bytes;
+  const int64_t vrow_bytes = VROW ? a.vs[2] * 2 : 0;
+  // Lane offset of load r: row = ROWS_PER_LOAD (NI w + r) + lane / CPR, whose
+  // swizzle is 4 r | lane / 16, so the chunk's byte is loff ^ 64 r.
+  const uint32_t lrow = G::ROWS_PER_LOAD * NI * w + lane / G::CPR;
+  const uint32_t loff = 16u * ((lane % G::CPR) ^ (lane >> 4));
   uint32_t koff[NI];
 #pragma unroll
   for (int r = 0; r < NI; ++r) koff[r] = k_lane_off<HD>(NI * w + r, lane, krow_bytes);
-  const int voff = w * NI * 1024 + 16 * lane;
+  const uint32_t vfirst = VROW ? lrow * static_cast<uint32_t>(vrow_bytes)
+                               : static_cast<uint32_t>(w * NI * 1024 + 16 * lane);
   // Loads 2 NI / NDS of the wave's 2 NI staging loads of block j (part
   // 0 .. NDS - 1).
   auto stage_part = [&](int j, u32x4* kst, u32x4* vst, int part) {
@@ -1128,21 +1139,38 @@ __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
     const int rows = Nk - j * BS < BS ? Nk - j * BS : BS;
     const sgpr_rsrc_t krs =
         make_sgpr_rsrc(kbytes + j * kblk_bytes, static_cast<uint32_t>(rows * krow_bytes));
-    const sgpr_rsrc_t vrs = make_sgpr_rsrc(vtbytes + static_cast<int64_t>(j) * TILE_BYTES, TILE_BYTES);
+    const sgpr_rsrc_t vrs =
+        VROW ? make_sgpr_rsrc(vtbytes + j * BS * vrow_bytes, static_cast<uint32_t>(rows * vrow_bytes))
+             : make_sgpr_rsrc(vtbytes + static_cast<int64_t>(j) * TILE_BYTES, TILE_BYTES);
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
       const int r = part * PER + q;
       if (r < NI)
         bdma16_untracked(krs, koff[r], 0u, kl + 1024 * r);
+      else if constexpr (VROW)
+        bdma16_untracked(vrs, vfirst + (loff ^ (64u * (r - NI))) +
+                                  static_cast<uint32_t>(G::ROWS_PER_LOAD * (r - NI)) *
+                                      static_cast<uint32_t>(vrow_bytes),
+                         0u, vl + 1024 * (r - NI));
       else
-        bdma16_untracked(vrs, voff + 1024u * (r - NI), 0u, vl + 1024 * (r - NI));
+        bdma16_untracked(vrs, vfirst + 1024u * (r - NI), 0u, vl + 1024 * (r - NI));
     }
   };
-  // K operand offset of (key tile kt, k-step ds) inside a K stage.
+  // K operand offset of (key tile 0, k-step 0) inside a K stage; k-step ds is
+  // at this ^ (64 ds).
+  uint32_t kread0 = G::ROW_BYTES * l16 + 16 * (g ^ G::kswz(l16));
   uint32_t kread[NDS];
 #pragma unroll
   for (int ds = 0; ds < NDS; ++ds)
     kread[ds] = G::ROW_BYTES * l16 + 16 * ((4 * ds + g) ^ G::kswz(l16));
+  // VROW: byte of V's row 4 g + l % 16 / 4, dims 4 (l % 4) .. + 3 of O^T tile 0
+  // inside a V stage; tile dt is at this ^ (32 dt) (the chunk swizzle is an
+  // XOR above the row's bits), key group s and half p at + 16 (2 s + p) rows.
+  uint32_t vread = 0;
+  if constexpr (VROW) {
+    const int vr = 4 * g + (l16 >> 2), cb = (l16 & 3) >> 1;
+    vread = static_cast<uint32_t>(G::ROW_BYTES * vr + 16 * (cb ^ G::kswz(vr)) + 8 * (l16 & 1));
+  }
   const uint32_t one2 = BF16 ? 0x3f803f80u : 0x3c003c00u;
   const u32x4 ones = {one2, one2, one2, one2};
 
@@ -1165,8 +1193,10 @@ __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
     auto read_k = [&](int ds, u32x4 (&dst)[4]) {
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt)
-        dst[kt] = *reinterpret_cast<const u32x4*>(ks + kread[ds] + TT_BYTES * kt);
+        dst[kt] = *reinterpret_cast<const u32x4*>(ks + (VROW ? kread0 ^ (64u * ds) : kread[ds]) + TT_BYTES * kt);
     };
+    // VROW: the other k-steps' offsets are formed per step; held, they spill.
+    if constexpr (VROW) asm volatile("" : "+v"(kread0));
     read_k(0, kf[0]);
 #pragma unroll
     for (int ds = 0; ds < NDS; ++ds) {
@@ -1186,12 +1216,22 @@ __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
     }
     // The first V^T operands are read before the softmax, the rest four
     // O^T tiles ahead of their MFMAs.
-    constexpr int VAHEAD = 4;
+    constexpr int VAHEAD = VROW ? 2 : 4;
     constexpr int PV_PART_EVERY = NDT / (NDS / 2);  // O^T tiles per staging part
     u32x4 vf[NDT][2];
     auto read_v = [&](int dt) {
-      vf[dt][0] = vts[(2 * dt + 0) * 64 + lane];
-      vf[dt][1] = vts[(2 * dt + 1) * 64 + lane];
+      if constexpr (VROW) {
+        const char* vb = reinterpret_cast<const char*>(vts) + (vread ^ (32u * dt));
+#pragma unroll
+        for (int ks2 = 0; ks2 < 2; ++ks2) {
+          const u32x2 lo = lds_read_tr16(vb + (32 * ks2) * G::ROW_BYTES);
+          const u32x2 hi = lds_read_tr16(vb + (32 * ks2 + 16) * G::ROW_BYTES);
+          vf[dt][ks2] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+        }
+      } else {
+        vf[dt][0] = vts[(2 * dt + 0) * 64 + lane];
+        vf[dt][1] = vts[(2 * dt + 1) * 64 + lane];
+      }
     };
 #pragma unroll
     for (int dt = 0; dt < VAHEAD; ++dt) read_v(dt);
@@ -1887,13 +1927,37 @@ struct AttnGeom {
   int list;
 };
 
+// Whether attn_pair_kernel takes a call.
+bool pair_path(cab_dtype_t dtype, const AttnGeom& g, int32_t kmax, bool sub) {
+  return dtype != CAB_F32 && !sub && pair_enabled() &&
+         ((g.list == LIST_LDS && kmax <= PAIR_KMAX) || g.list == LIST_DENSE);
+}
+// ... and reads V's rows instead of tiles packed ahead of it: where a key block
+// is visited `visits` times on average, at most V_ROW_VISITS. The packing pass
+// costs a launch and two passes over V (155 us at 32 heads x 65536 keys), the
+// transposing reads 3-8 % of the kernel. bf16, causal, packed -> rows, us:
+// lists of 3 of 4000 keys (32 heads) 48.5 -> 38.2, of 24 of 16000 460 -> 438, of
+// 31 of 40000 1405 -> 1382, of 62 2411 -> 2455; dense 500 keys (12 heads) 19.5 ->
+// 15.8, 1000 (32 heads on 8, 31 visits) 29.9 -> 26.2, 2000 (62) 58.4 -> 57.9, 9000
+// (281) 612 -> 631. 64 rows are addressed by 32-bit offsets.
+constexpr int64_t V_ROW_VISITS = 48;
+bool v_rows(const int64_t* v_strides, int64_t visits) {
+  return visits <= V_ROW_VISITS && v_strides[2] <= (int64_t{1} << 24);
+}
+// A dense call's visits per key block of one K / V head, causal or not.
+int64_t dense_visits(const AttnGeom& g, int causal) {
+  const int64_t mq = ceil_div(g.Nq, BS), mk = ceil_div(g.Nk, BS), all = g.H / g.Hkv * mq;
+  return causal && mk > 0 ? all * (2 * mk - (mq < mk ? mq : mk)) / (2 * mk) : all;
+}
+
 cab_status_t launch_attn(const char* fn, const void* q, const void* k, const void* vt,
                          cab_dtype_t dtype, const AttnGeom& g, const int64_t* q_strides,
                          const int64_t* k_strides, const int64_t* o_strides,
                          const int32_t* kv_idx, const int32_t* kv_cnt, int32_t kmax, float scale,
                          int causal, void* out, float* lse, hipStream_t s,
                          const uint64_t* submask = nullptr, int sub_shift = 0, int splits = 1,
-                         float* parts = nullptr) {
+                         float* parts = nullptr, const void* v = nullptr,
+                         const int64_t* v_strides = nullptr) {
   const int64_t M = ceil_div(g.Nq, BS);
   AttnArgs a;
   a.q = q;
@@ -1905,7 +1969,9 @@ cab_status_t launch_attn(const char* fn, const void* q, const void* k, const voi
     a.qs[d] = q_strides[d];
     a.ks[d] = k_strides[d];
     a.os[d] = o_strides[d];
+    a.vs[d] = v_strides ? v_strides[d] : 0;
   }
+  a.v = static_cast<const uint16_t*>(v);
   a.kv_idx = kv_idx;
   a.kv_cnt = kv_cnt;
   a.BH = static_cast<int32_t>(g.B * g.H);
@@ -1924,22 +1990,29 @@ cab_status_t launch_attn(const char* fn, const void* q, const void* k, const voi
   a.splits = splits;
   a.po = parts;
   a.pml = parts ? parts + static_cast<int64_t>(splits) * a.BH * a.N * g.D : nullptr;
-  if (dtype != CAB_F32 && submask == nullptr && pair_enabled() &&
-      ((g.list == LIST_LDS && kmax <= PAIR_KMAX) || g.list == LIST_DENSE)) {
+  if (pair_path(dtype, g, kmax, submask != nullptr)) {
     const dim3 pgrid(static_cast<unsigned>(g.B * g.H * ((M + 1) / 2)));
     auto go = [&](auto dt_tag, auto hd_tag) {
       constexpr cab_dtype_t DT = decltype(dt_tag)::value;
       constexpr int HD = decltype(hd_tag)::value;
-      if (g.list == LIST_DENSE && splits > 1) {
-        const dim3 sgrid(pgrid.x * static_cast<unsigned>(splits));
-        attn_pair_kernel<DT, LIST_DENSE_SPLIT, HD><<<sgrid, 256, 0, s>>>(a);
-        const int64_t per = 256 / (HD / 4);
-        split_combine_kernel<DT == CAB_BF16, HD>
-            <<<static_cast<unsigned>(ceil_div(static_cast<int64_t>(a.BH) * a.N, per)), 256, 0, s>>>(a);
-      } else if (g.list == LIST_DENSE)
-        attn_pair_kernel<DT, LIST_DENSE, HD><<<pgrid, 256, 0, s>>>(a);
+      auto with_v = [&](auto rows_tag) {
+        constexpr bool VROW = decltype(rows_tag)::value;
+        if (g.list == LIST_DENSE && splits > 1) {
+          const dim3 sgrid(pgrid.x * static_cast<unsigned>(splits));
+          attn_pair_kernel<DT, LIST_DENSE_SPLIT, HD, VROW><<<sgrid, 256, 0, s>>>(a);
+          const int64_t per = 256 / (HD / 4);
+          split_combine_kernel<DT == CAB_BF16, HD>
+              <<<static_cast<unsigned>(ceil_div(static_cast<int64_t>(a.BH) * a.N, per)), 256, 0, s>>>(a);
+        } else if (g.list == LIST_DENSE) {
+          attn_pair_kernel<DT, LIST_DENSE, HD, VROW><<<pgrid, 256, 0, s>>>(a);
+        } else {
+          attn_pair_kernel<DT, LIST_LDS, HD, VROW><<<pgrid, 256, 0, s>>>(a);
+        }
+      };
+      if (v)
+        with_v(std::true_type{});
       else
-        attn_pair_kernel<DT, LIST_LDS, HD><<<pgrid, 256, 0, s>>>(a);
+        with_v(std::false_type{});
     };
     using BF = std::integral_constant<cab_dtype_t, CAB_BF16>;
     using FH = std::integral_constant<cab_dtype_t, CAB_F16>;
@@ -2123,12 +2196,16 @@ extern "C" cab_status_t cab_block_sparse_attn_fwd(
     }
     if ((st = launch_status("cab_block_sparse_attn_fwd/relist")) != CAB_OK) return st;
   }
+  const int32_t k64 = block_size == BS ? kmax : static_cast<int32_t>(tl.K64);
+  const bool vrows = v_rows(v_strides, k64) &&
+                     pair_path(dtype, sparse_geom(B, H, N, D, k64), k64, block_size < BS);
   if (dtype == CAB_F32)
     st = launch_pack_split("cab_block_sparse_attn_fwd/pack_split", k, k_strides, v, v_strides, B,
                            H, N, D, workspace, s);
-  else
+  else if (!vrows)
     st = launch_pack("cab_block_sparse_attn_fwd/pack_v", v, v_strides, B, H, N, D, workspace, s);
   if (st != CAB_OK) return st;
+  const void* vp = vrows ? v : nullptr;
   if (block_size != BS) {
     const char* ws = static_cast<const char*>(workspace);
     int sh = 0;
@@ -2139,10 +2216,11 @@ extern "C" cab_status_t cab_block_sparse_attn_fwd(
                        reinterpret_cast<const int32_t*>(ws + tl.off_cnt),
                        static_cast<int32_t>(tl.K64), scale, causal, out, lse, s,
                        block_size < BS ? reinterpret_cast<const uint64_t*>(ws + tl.off_sub) : nullptr,
-                       sh);
+                       sh, 1, nullptr, vp, v_strides);
   }
   return launch_attn(fn, q, k, workspace, dtype, sparse_geom(B, H, N, D, kmax), q_strides, k_strides,
-                     o_strides, kv_idx, kv_cnt, kmax, scale, causal, out, lse, s);
+                     o_strides, kv_idx, kv_cnt, kmax, scale, causal, out, lse, s, nullptr, 0, 1, nullptr,
+                     vp, v_strides);
 }
 
 // ---------------------------------------------------------------------------
@@ -2351,16 +2429,18 @@ cab_status_t dense_forward(const char* fn, const void* q, const void* k, const v
   if (scores && !lse)
     lse = reinterpret_cast<float*>(static_cast<char*>(workspace) + plan.off_lse);
   if (scores && (st = check_score_rows(fn, q, lse, q_strides, esize)) != CAB_OK) return st;
+  const AttnGeom g{B, H, H_kv, N_q, N_k, D, N_k - N_q, LIST_DENSE};
+  const bool vrows = v_rows(v_strides, dense_visits(g, causal)) && pair_path(dtype, g, 1, false);
   if (dtype == CAB_F32)
     st = launch_pack_split(fn, k, k_strides, v, v_strides, B, H_kv, N_k, D, workspace, s);
-  else
+  else if (!vrows)
     st = launch_pack(fn, v, v_strides, B, H_kv, N_k, D, workspace, s);
   if (st != CAB_OK) return st;
-  const AttnGeom g{B, H, H_kv, N_q, N_k, D, N_k - N_q, LIST_DENSE};
   st = launch_attn(fn, q, k, workspace, dtype, g, q_strides, k_strides, o_strides, nullptr,
                    nullptr, 1, scale, causal, out, lse, s, nullptr, 0, plan.splits,
                    plan.splits > 1 ? reinterpret_cast<float*>(static_cast<char*>(workspace) + plan.off_parts)
-                                   : nullptr);
+                                   : nullptr,
+                   vrows ? v : nullptr, v_strides);
   if (st != CAB_OK || !scores) return st;
   return launch_key_scores(fn, q, k, lse, dtype, B, H, H_kv, N_q, N_k, D, q_strides, k_strides,
                            scale, causal, t, s);
