@@ -194,6 +194,15 @@ def aligned_rows(t: torch.Tensor) -> torch.Tensor:
     return t if rows_aligned(t) else t.clone()
 
 
+def addressable(*tensors: torch.Tensor) -> bool:
+    """Whether a kernel may stand in for torch ops on ``tensors``: plain tensors,
+    with no transform (vmap, forward-mode, tracing) that has to see the ops."""
+    return (all(type(t) is torch.Tensor or type(t) is torch.nn.Parameter for t in tensors)
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and torch.autograd.forward_ad._current_level < 0
+            and not torch.compiler.is_compiling() and not torch.jit.is_tracing())
+
+
 _SAME_DEVICE = contextlib.nullcontext()
 
 

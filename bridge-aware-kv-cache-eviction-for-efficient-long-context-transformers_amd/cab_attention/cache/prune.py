@@ -24,10 +24,10 @@ def append_rows(k: torch.Tensor, v: torch.Tensor, k_dst: torch.Tensor, v_dst: to
     """Copies ``k``, ``v`` ``[B, H, n, D]`` to rows ``row ..`` of the buffers
     ``[B, H, capacity, >= D]`` (one stride set, contiguous last dim) in one
     launch (``cab_kv_append``). False, and nothing done, for what the kernel
-    does not take (another device or dtype, gradients to record)."""
+    does not take (another device or dtype, gradients to record, a transform)."""
     dev = k_dst.device
     if (dev.type != "cuda" or k.device != dev or v.device != dev
-            or k.dtype not in _APPEND_DTYPES or k_dst.dtype != k.dtype
+            or not nat.addressable(k, v, k_dst, v_dst) or k.dtype not in _APPEND_DTYPES or k_dst.dtype != k.dtype
             or (torch.is_grad_enabled() and (k.requires_grad or v.requires_grad
                                              or k_dst.requires_grad or v_dst.requires_grad))):
         return False

@@ -49,7 +49,7 @@ class ImportanceTracker:
         included. False, and nothing done, for what it does not take."""
         old = self.cumulative_scores
         if (w.device.type != "cuda" or w.dim() != 4 or w.dtype not in _DTYPES or w.numel() == 0
-                or (w.requires_grad and torch.is_grad_enabled())):
+                or (w.requires_grad and torch.is_grad_enabled()) or not nat.addressable(w)):
             return False
         B, H, n_q, n_k = w.shape
         if old is None:

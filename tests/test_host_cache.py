@@ -170,3 +170,16 @@ def test_cache_views_are_read_only_and_alias_the_store(monkeypatch):
         cache.update(y, y, 0, None)
     assert cache.total_evictions >= 2
     assert not torch.equal(kept, snapshot)  # the old view now shows a later prune's rows
+
+
+def test_kernels_leave_transforms_to_torch():
+    from cab_attention import _native as nat
+    x = torch.zeros(2, 3)
+    seen = []
+    assert nat.addressable(x, torch.nn.Parameter(x))
+    torch.vmap(lambda r: (seen.append(nat.addressable(r)), r)[1])(x)
+    with torch.autograd.forward_ad.dual_level():
+        seen.append(nat.addressable(torch.autograd.forward_ad.make_dual(x, x)))
+    seen.append(nat.addressable(x.as_subclass(type("Sub", (torch.Tensor,), {}))))
+    torch.jit.trace(lambda r: (seen.append(nat.addressable(r)), r + 1)[1], x, check_trace=False)
+    assert seen == [False] * 4
