@@ -1262,23 +1262,25 @@ __global__ __launch_bounds__(WI * WJ * 64, 1) void triangle_kernel(TriArgs a) {
 // (b, h). Wave w owns the 32 x 32 tile (w / 4, w % 4) of A, of Ahat and of T alike:
 //   A = alpha Qc Kc^T, operands straight from global memory;
 //   min / max through LDS;
-//   Ahat stays in registers in fp32, X = f16(Ahat) goes to LDS row-major and
-//   transposed (the two MFMA operands; zero past M);
-//   T = X X with fp32 accumulate, and F from Ahat and T in registers.
+//   X = f16(Ahat) goes to LDS row-major and X, or the fused form's
+//   I - lambda X, transposed (the two MFMA operands; zero past M);
+//   T (or, fused, F) with fp32 accumulate, and F from Ahat and T in registers.
 // Against STATS, EMIT, (min / max) and the triangle kernel this saves two or
 // three launches and the planes' round trip; launch and load latency bound it.
 // cab_block_frc, (b, h) x M x D, general path -> here: 8 x 16 x 128 fp16 18.9 -> 5.8
 // us, 8 x 128 x 128 bf16 17.8 -> 15.1, 512 x 128 x 128 bf16 43.5 -> 33.6, 16 x 64 x 64
 // fp32 42.8 -> 8.7, 32 x 128 x 128 fp32 with diagnostics 84.5 -> 22.9.
-// Numerics as on the large path: one fp16 product per site for T; Ahat in F at
-// fp32 accuracy (the fused additive form rounds it to fp16).
+// The roundings are those of the other kernels, and so are the orders of the
+// sums (one accumulator per element, k ascending, the same MFMA): F, and with it
+// the choice of blocks, comes out bit for bit as theirs.
 // ---------------------------------------------------------------------------
 constexpr int SMALL_M = 128;
 
 struct SmallArgs {
   const void* qc;
   const void* kc;
-  int32_t M, D, formula;
+  int32_t M, D, formula, fused;
+  int32_t recip;  // normalise by 1 / (max - min + 1e-8), as aff_strip_kernel does
   float alpha, lambda;
   float* frc;
   float* affinity;   // or null
@@ -1360,17 +1362,26 @@ __global__ __launch_bounds__(1024) void frc_small_kernel(SmallArgs a) {
   }
   // A constant A stays as it is (outside fp16's range, perhaps): T = M c^2 below.
   const bool constant = !(mx > mn);
+  const float recip = 1.0f / (mx - mn + 1e-8f);
 #pragma unroll
   for (int e = 0; e < 16; ++e) {
     const bool in = i0 + row_of(e) < M && j < M;
-    acc[e] = in ? normalize_minmax(acc[e], mn, mx) : 0.f;
+    const float v = a.recip && !constant ? (acc[e] - mn) * recip : normalize_minmax(acc[e], mn, mx);
+    acc[e] = in ? v : 0.f;
     xs[i0 + row_of(e)][j] = constant ? uint16_t{0} : f32_to_f16(acc[e]);
   }
 #pragma unroll
   for (int e = 0; e < 16; e += 4) {
     uint16_t h[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) h[q] = constant ? uint16_t{0} : f32_to_f16(acc[e + q]);
+    for (int q = 0; q < 4; ++q) {
+      const int i = i0 + row_of(e + q);
+      const float d = i == j && i < M ? 1.f : 0.f;
+      // (each conversion in its own arm: d - lambda Ahat is then rounded once, by a
+      // mixed-precision fma, as in the other kernels)
+      const uint16_t x = a.fused ? f32_to_f16(d - a.lambda * acc[e + q]) : f32_to_f16(acc[e + q]);
+      h[q] = constant ? uint16_t{0} : x;
+    }
     *reinterpret_cast<u32x2*>(&xt[j][i0 + row_of(e)]) =
         u32x2{h[0] | static_cast<uint32_t>(h[1]) << 16, h[2] | static_cast<uint32_t>(h[3]) << 16};
   }
@@ -1389,7 +1400,17 @@ __global__ __launch_bounds__(1024) void frc_small_kernel(SmallArgs a) {
     const int r = row_of(e);
     if (i0 + r >= M) continue;
     const float tv = constant ? static_cast<float>(M) * acc[e] * acc[e] : t[e];
-    a.frc[base + r * M] = frc_combine(a.formula, acc[e], tv, a.lambda, 0.f, 0.f);
+    if (a.fused && !constant) {
+      a.frc[base + r * M] = isfinite(tv) ? tv : 0.f;
+    } else {
+      // Ahat as the planes hold it: f16, plus its f16 remainder where F is a quotient.
+      float ahat = acc[e];
+      if (!constant) {
+        const float hi = f16_to_f32(f32_to_f16(ahat));
+        ahat = a.formula == CAB_FRC_ADDITIVE ? hi : hi + f16_to_f32(f32_to_f16(ahat - hi));
+      }
+      a.frc[base + r * M] = frc_combine(a.formula, ahat, tv, a.lambda, 0.f, 0.f);
+    }
     if (a.affinity) a.affinity[base + r * M] = acc[e];
     if (a.triangles) a.triangles[base + r * M] = tv;
   }
@@ -1528,8 +1549,9 @@ extern "C" cab_status_t cab_block_frc(const void* qc, const void* kc, cab_dtype_
   a.strip = 1;
 
   if (f16 && M <= SMALL_M) {
-    const SmallArgs sa{qc, kc, static_cast<int32_t>(M), static_cast<int32_t>(D), formula, a.alpha,
-                       lambda_redundancy, frc, affinity, triangles};
+    const SmallArgs sa{qc, kc, static_cast<int32_t>(M), static_cast<int32_t>(D), formula, fused ? 1 : 0,
+                       strip_path(dtype, D) ? 1 : 0, a.alpha, lambda_redundancy, frc, affinity,
+                       triangles};
     const unsigned grid = static_cast<unsigned>(BH);
     switch (dtype) {
       case CAB_BF16: frc_small_kernel<bf16_t><<<grid, 1024, 0, s>>>(sa); break;

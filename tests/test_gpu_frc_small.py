@@ -50,3 +50,22 @@ def test_constant_affinity(cuda):
     torch.testing.assert_close(aff.cpu(), torch.full((1, 1, 50, 50), c))
     torch.testing.assert_close(tri.cpu(), torch.full((1, 1, 50, 50), 50 * c * c))
     torch.testing.assert_close(frc.cpu(), torch.full((1, 1, 50, 50), c - 0.5 * 50 * c * c))
+
+
+@pytest.mark.parametrize("M", [16, 33, 100, 128, 129])
+@pytest.mark.parametrize("dt", ["bf16", "fp16", "fp32"])
+def test_fused_form_has_one_set_of_roundings(cuda, M, dt):
+    """Without diagnostics F = X (I - lambda X)^T of fp16 planes, at M <= 128 as
+    above it: blocks at the selection's threshold do not depend on M's side of 128."""
+    from cab_attention.kernels import compute_block_frc
+    g = torch.Generator().manual_seed(M)
+    qc, kc = (torch.randn((1, 2, M, 64), generator=g).to(DTYPES[dt]).to(cuda) for _ in range(2))
+    lam = float(np.float32(0.7))
+    _, aff, _ = compute_block_frc(qc, kc, lambda_redundancy=lam)
+    frc, _, _ = compute_block_frc(qc, kc, lambda_redundancy=lam, diagnostics=False)
+    a = aff.cpu().double()
+    x = a.half().double()
+    xt = (torch.eye(M, dtype=torch.float64) - lam * a).half().double()  # [k][j], rounded once
+    want = torch.matmul(x, xt)
+    bound = M * 2.0 ** -23 * torch.matmul(x.abs(), xt.abs()) + 1e-9  # fp32 sums of exact products
+    assert bool(((frc.cpu().double() - want).abs() <= bound).all())
