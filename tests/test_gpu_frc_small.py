@@ -1,5 +1,5 @@
-"""compute_block_frc at M <= 128 (one kernel) and 129 (the general ones), at
-the edges of its 32-wide tiles and 16-deep k-steps, every input type and
+"""compute_block_frc at M <= 128 (one kernel) and above (the general ones: the
+affinity's runs of four columns whole and cut), at the edges of 32-wide tiles and 16-deep k-steps, every input type and
 formula it takes, with and without diagnostics, against the oracle."""
 
 import numpy as np
@@ -14,7 +14,8 @@ DTYPES = {"bf16": torch.bfloat16, "fp16": torch.float16, "fp32": torch.float32}
 
 
 @pytest.mark.parametrize("M,D", [(1, 128), (2, 8), (31, 64), (32, 24), (33, 128), (64, 256), (65, 72),
-                                 (100, 128), (127, 64), (128, 128), (129, 128)])
+                                 (100, 128), (127, 64), (128, 128), (129, 128),
+                                 (130, 64), (131, 128), (132, 72), (255, 128)])
 @pytest.mark.parametrize("dt", ["bf16", "fp16", "fp32"])
 @pytest.mark.parametrize("formula", ["additive", "multiplicative"])
 def test_frc_small(cuda, M, D, dt, formula):
