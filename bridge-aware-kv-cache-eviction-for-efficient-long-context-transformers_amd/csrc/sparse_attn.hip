@@ -1367,7 +1367,9 @@ __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
 
 // Merges the splits of attn_pair_kernel<LIST_DENSE_SPLIT>: HD / 4 threads per
 // query, each four output values. A split in which the query has no key has
-// l = 0 and is skipped.
+// l = 0 and is skipped; a NaN sum (a NaN or a score of +inf in that split) is
+// not, so the query's output is NaN as it is unsplit. The sum's bits are
+// tested because this file is compiled with -fno-honor-nans.
 template <bool BF16, int HD>
 __global__ __launch_bounds__(256) void split_combine_kernel(AttnArgs a) {
   constexpr int TD = HD / 4;
@@ -1385,7 +1387,7 @@ __global__ __launch_bounds__(256) void split_combine_kernel(AttnArgs a) {
     const float ls = pl[s * rows + row];
     const float f = __builtin_amdgcn_exp2f((a.pml[s * rows + row] - m) * a.scale_log2);
     const f32x4 x = reinterpret_cast<const f32x4*>(a.po + (s * rows + row) * HD)[d4];
-    if (ls > 0.f) {
+    if (__float_as_uint(ls) != 0u) {
       l += ls * f;
       o += x * f;
     }
