@@ -375,6 +375,7 @@ struct CombineArgs {
   const float* s;
   int64_t ld;
   int32_t H, Nq, Nk, splits;
+  int32_t qoff, causal;
   float c;
   char* out;
   int64_t os[3];  // bytes
@@ -435,19 +436,25 @@ __global__ __launch_bounds__(256) void row_combine_kernel(CombineArgs a) {
       const int64_t row = (static_cast<int64_t>(bh) * a.Nq + t) * a.splits;
       float m, l;
       merge_row(a.pm + row, a.pl + row, a.splits, c, m, l);
-      // (a query without keys adds nothing)
-      if (lane_id() == 0) lse2[t] = l > 0.f ? m * c + __log2f(l) : INFINITY;
+      // (a query without keys adds nothing; one whose sum is NaN makes the totals of
+      // the keys it sees NaN, and of no others)
+      if (lane_id() == 0) lse2[t] = l == 0.f ? INFINITY : m * c + __log2f(l);
     }
     __syncthreads();
+    // Keys query t does not see hold scores of -inf; they add 0 whatever its lse.
+    const int see = a.causal ? a.qoff + 1 : a.Nk;  // + t where causal
     float sum[PER];
 #pragma unroll
-    for (int i = 0; i < PER; ++i) sum[i] = __builtin_amdgcn_exp2f(sv[i] - lse2[0]);
+    for (int i = 0; i < PER; ++i)
+      sum[i] = key0 + 256 * i < see ? __builtin_amdgcn_exp2f(sv[i] - lse2[0]) : 0.f;
 #pragma unroll 4
     for (int t = 1; t < a.Nq; ++t) {
+      const int lim = a.causal ? see + t : see;
 #pragma unroll
       for (int i = 0; i < PER; ++i) {
         const int key = key0 + 256 * i;  // (past the keys: a key of the row, not stored)
-        sum[i] += __builtin_amdgcn_exp2f(srow[t * a.ld + (key < a.Nk ? key : 0)] - lse2[t]);
+        const float p = __builtin_amdgcn_exp2f(srow[t * a.ld + (key < a.Nk ? key : 0)] - lse2[t]);
+        sum[i] += key < lim ? p : 0.f;
       }
     }
     float* drow = a.scores + b * a.ss[0] + h * a.ss[1];
@@ -585,6 +592,8 @@ cab_status_t row_attn_launch(const char* fn, const RowAttnProblem& p, void* ws, 
   ca.Nq = a.Nq;
   ca.Nk = a.Nk;
   ca.splits = a.splits;
+  ca.qoff = a.qoff;
+  ca.causal = a.causal;
   ca.c = a.c;
   ca.out = static_cast<char*>(p.out);
   ca.lse = p.lse;

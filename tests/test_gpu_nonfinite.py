@@ -1,6 +1,6 @@
 """NaN and infinities in q, k and v of the dense calls: the outputs and key
-totals that are not finite are those a float64 softmax has, whether the key
-blocks are split (into two and into four parts) or not."""
+totals that are not finite are those a float64 softmax has, whichever kernels
+run (few rows, the key blocks split into two and into four parts, unsplit)."""
 
 import pytest
 import torch
@@ -9,6 +9,9 @@ pytestmark = pytest.mark.gpu
 
 DTYPES = {"bf16": torch.bfloat16, "fp16": torch.float16, "fp32": torch.float32}
 ROUTES = [  # (H, H_kv, N_q, N_k)
+    (4, 2, 3, 200),     # few rows
+    (8, 2, 1, 700),
+    (4, 4, 24, 1100),
     (2, 2, 33, 1281),   # key blocks in two parts (16-bit types), the last holds one key
     (4, 2, 100, 2700),  # four parts
     (4, 2, 100, 300),   # one part
