@@ -704,6 +704,11 @@ __global__ __launch_bounds__(256, DT == CAB_F32 ? 1 : 2) void attn_fwd_kernel(At
   // bytes).
   const int64_t krow_bytes = a.ks[2] * 2;
   const int64_t kblk_bytes = BS * krow_bytes;
+  // Bytes of block j's valid rows: to the end of the last one, which lies past
+  // rows * krow_bytes where rows overlap (a token stride below D).
+  const uint32_t kfull = static_cast<uint32_t>((BS - 1) * krow_bytes + 2 * HD);
+  const uint32_t klast = static_cast<uint32_t>((Nk - 1) % BS * krow_bytes + 2 * HD);
+  auto k_bytes = [&](int j) { return j + 1 < Mk ? kfull : klast; };
   uint32_t koff[NI];
 #pragma unroll
   for (int r = 0; r < NI; ++r) koff[r] = k_lane_off<HD>(NI * w + r, ge.lane, krow_bytes);
@@ -712,8 +717,7 @@ __global__ __launch_bounds__(256, DT == CAB_F32 ? 1 : 2) void attn_fwd_kernel(At
   auto stage_part = [&](int j, u32x4* kst, u32x4* vst, int ds) {
     constexpr int PER = 2 * NI / G::NDS;
     char* kl = reinterpret_cast<char*>(kst) + w * NI * 1024;
-    const int rows = Nk - j * BS < BS ? Nk - j * BS : BS;
-    const brsrc_t krs = make_rsrc(kbytes + j * kblk_bytes, static_cast<uint32_t>(rows * krow_bytes));
+    const brsrc_t krs = make_rsrc(kbytes + j * kblk_bytes, k_bytes(j));
     const brsrc_t vrs = make_rsrc(vtbytes + static_cast<int64_t>(j) * TILE_BYTES, TILE_BYTES);
     char* vl = reinterpret_cast<char*>(vst) + w * NI * 1024;
 #pragma unroll
@@ -739,8 +743,7 @@ __global__ __launch_bounds__(256, DT == CAB_F32 ? 1 : 2) void attn_fwd_kernel(At
       return;
     }
     char* kl = reinterpret_cast<char*>(kst) + w * NI * 1024;
-    const int rows = Nk - j * BS < BS ? Nk - j * BS : BS;
-    const brsrc_t krs = make_rsrc(kbytes + j * kblk_bytes, static_cast<uint32_t>(rows * krow_bytes));
+    const brsrc_t krs = make_rsrc(kbytes + j * kblk_bytes, k_bytes(j));
 #pragma unroll
     for (int r = 0; r < NI; ++r) bdma16(krs, koff[r], 0, kl + 1024 * r);
     const brsrc_t vrs = make_rsrc(vtbytes + static_cast<int64_t>(j) * TILE_BYTES, TILE_BYTES);
@@ -1120,6 +1123,12 @@ __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
   const int64_t krow_bytes = a.ks[2] * 2;
   const int64_t kblk_bytes = BS * krow_bytes;
   const int64_t vrow_bytes = VROW ? a.vs[2] * 2 : 0;
+  // Descriptor sizes of a whole block and of the last one (see attn_fwd_kernel).
+  const int last_row = (Nk - 1) % BS;
+  const uint32_t kfull = static_cast<uint32_t>((BS - 1) * krow_bytes + 2 * HD);
+  const uint32_t klast = static_cast<uint32_t>(last_row * krow_bytes + 2 * HD);
+  const uint32_t vfull = static_cast<uint32_t>((BS - 1) * vrow_bytes + 2 * HD);
+  const uint32_t vlast = static_cast<uint32_t>(last_row * vrow_bytes + 2 * HD);
   // Lane offset of load r: row = ROWS_PER_LOAD (NI w + r) + lane / CPR, whose
   // swizzle is 4 r | lane / 16, so the chunk's byte is loff ^ 64 r.
   const uint32_t lrow = G::ROWS_PER_LOAD * NI * w + lane / G::CPR;
@@ -1136,11 +1145,10 @@ __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
     static_assert(NDS % 2 == 0 && NDT % (NDS / 2) == 0, "staging parts split over S and P V");
     char* kl = reinterpret_cast<char*>(kst) + w * NI * 1024;
     char* vl = reinterpret_cast<char*>(vst) + w * NI * 1024;
-    const int rows = Nk - j * BS < BS ? Nk - j * BS : BS;
-    const sgpr_rsrc_t krs =
-        make_sgpr_rsrc(kbytes + j * kblk_bytes, static_cast<uint32_t>(rows * krow_bytes));
+    const bool whole = j + 1 < Mk;
+    const sgpr_rsrc_t krs = make_sgpr_rsrc(kbytes + j * kblk_bytes, whole ? kfull : klast);
     const sgpr_rsrc_t vrs =
-        VROW ? make_sgpr_rsrc(vtbytes + j * BS * vrow_bytes, static_cast<uint32_t>(rows * vrow_bytes))
+        VROW ? make_sgpr_rsrc(vtbytes + j * BS * vrow_bytes, whole ? vfull : vlast)
              : make_sgpr_rsrc(vtbytes + static_cast<int64_t>(j) * TILE_BYTES, TILE_BYTES);
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
@@ -1652,7 +1660,8 @@ __global__ __launch_bounds__(64 * NW) void key_score_kernel(KeyScoreArgs a) {
     const int q0 = 16 * tile_of(it);
     const uint32_t rows = static_cast<uint32_t>(min(16, a.Nq - q0));
     if (qstager) {
-      const brsrc_t qrs = make_rsrc(qb + static_cast<int64_t>(q0) * a.qs[2] * ESZ, rows * qrow);
+      const brsrc_t qrs =
+          make_rsrc(qb + static_cast<int64_t>(q0) * a.qs[2] * ESZ, (rows - 1) * qrow + HD * ESZ);
       if constexpr (F32) {
         bdma16(qrs, q_voff, 0, st + 2048 * w);
         bdma16(qrs, q_voff + 16u, 0, st + 2048 * w + 1024);
@@ -1943,8 +1952,10 @@ bool pair_path(cab_dtype_t dtype, const AttnGeom& g, int32_t kmax, bool sub) {
 // 15.8, 1000 (32 heads on 8, 31 visits) 29.9 -> 26.2, 2000 (62) 58.4 -> 57.9, 9000
 // (281) 612 -> 631. 64 rows are addressed by 32-bit offsets.
 constexpr int64_t V_ROW_VISITS = 48;
-bool v_rows(const int64_t* v_strides, int64_t visits) {
-  return visits <= V_ROW_VISITS && v_strides[2] <= (int64_t{1} << 24);
+// Rows that overlap (a token stride below D, an expanded row) are packed: the
+// descriptor could not tell a row past the keys from the valid ones.
+bool v_rows(const int64_t* v_strides, int64_t D, int64_t visits) {
+  return visits <= V_ROW_VISITS && v_strides[2] >= D && v_strides[2] <= (int64_t{1} << 24);
 }
 // A dense call's visits per key block of one K / V head, causal or not.
 int64_t dense_visits(const AttnGeom& g, int causal) {
@@ -2199,7 +2210,7 @@ extern "C" cab_status_t cab_block_sparse_attn_fwd(
     if ((st = launch_status("cab_block_sparse_attn_fwd/relist")) != CAB_OK) return st;
   }
   const int32_t k64 = block_size == BS ? kmax : static_cast<int32_t>(tl.K64);
-  const bool vrows = v_rows(v_strides, k64) &&
+  const bool vrows = v_rows(v_strides, D, k64) &&
                      pair_path(dtype, sparse_geom(B, H, N, D, k64), k64, block_size < BS);
   if (dtype == CAB_F32)
     st = launch_pack_split("cab_block_sparse_attn_fwd/pack_split", k, k_strides, v, v_strides, B,
@@ -2432,7 +2443,7 @@ cab_status_t dense_forward(const char* fn, const void* q, const void* k, const v
     lse = reinterpret_cast<float*>(static_cast<char*>(workspace) + plan.off_lse);
   if (scores && (st = check_score_rows(fn, q, lse, q_strides, esize)) != CAB_OK) return st;
   const AttnGeom g{B, H, H_kv, N_q, N_k, D, N_k - N_q, LIST_DENSE};
-  const bool vrows = v_rows(v_strides, dense_visits(g, causal)) && pair_path(dtype, g, 1, false);
+  const bool vrows = v_rows(v_strides, D, dense_visits(g, causal)) && pair_path(dtype, g, 1, false);
   if (dtype == CAB_F32)
     st = launch_pack_split(fn, k, k_strides, v, v_strides, B, H_kv, N_k, D, workspace, s);
   else if (!vrows)

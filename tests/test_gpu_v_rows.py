@@ -84,3 +84,57 @@ def test_v_rows_far_apart(cuda):
                        flash_attention(q, k, far, causal=True))
     want, _, _ = O.dense_attention_scores(*(x.astype(np.float64) for x in f), causal=True)
     assert np.abs(flash_attention(q, k, far, causal=True).float().cpu().numpy() - want).max() <= ATOL["bf16"]
+
+
+def _short_rows(x, stride):
+    """Random values in x's shape, dtype and place, with a token stride below D:
+    rows that overlap, or one row for all of them (stride 0)."""
+    _, H, N, D = x.shape
+    flat = torch.randn((1, H, (N - 1) * stride + D), generator=torch.Generator().manual_seed(N + D))
+    flat = flat.to(x.dtype).to(x.device)
+    return flat.as_strided((1, H, N, D), (flat.stride(0), flat.stride(1), stride, 1))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("dt", ["bf16", "fp16"])
+@pytest.mark.parametrize("stride", [0, 16, 56])
+@pytest.mark.parametrize("which", ["q", "k", "v"])
+@pytest.mark.parametrize("H,Hkv,Nq,Nk,causal", [
+    (2, 2, 100, 100, True), (2, 1, 65, 1500, True), (2, 2, 40, 1300, False),
+    (4, 1, 2000, 1600, False),  # 128 visits: packed
+    (2, 2, 3, 400, True),       # few rows
+])
+def test_dense_rows_closer_than_their_length(cuda, H, Hkv, Nq, Nk, causal, which, stride, dt, D):
+    """Token strides below D (an expanded row, overlapping windows) read the same
+    rows as a contiguous copy: output and key totals."""
+    from cab_attention.kernels import flash_attention_with_cumulative_scores
+    qkv, _ = _qkv(H, Hkv, Nq, Nk, D, dt, "plain", cuda)
+    at = "qkv".index(which)
+    qkv = list(qkv)
+    qkv[at] = _short_rows(qkv[at], stride)
+    want, _, want_sc = O.dense_attention_scores(
+        *(x.double().cpu().numpy() for x in qkv), causal=causal)
+    out, sc = flash_attention_with_cumulative_scores(*qkv, causal=causal)
+    assert np.abs(out.double().cpu().numpy() - want).max() <= ATOL[dt]
+    np.testing.assert_allclose(sc.double().cpu().numpy(), want_sc, rtol=1e-2, atol=1e-4)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("which", ["q", "k", "v"])
+@pytest.mark.parametrize("stride", [0, 16])
+@pytest.mark.parametrize("N,kmax,bs", [(1000, 5, 64), (64 * 50, 49, 64), (1500, 3, 128), (700, 8, 32)])
+def test_lists_rows_closer_than_their_length(cuda, N, kmax, bs, stride, which, D):
+    from cab_attention.kernels import block_sparse_attention
+    qkv, _ = _qkv(2, 2, N, N, D, "bf16", "plain", cuda)
+    at = "qkv".index(which)
+    qkv = list(qkv)
+    qkv[at] = _short_rows(qkv[at], stride)
+    M = (N + bs - 1) // bs
+    rng = np.random.default_rng(N)
+    idx = np.stack([np.sort(rng.permutation(M)[:kmax]) for _ in range(2 * M)])
+    idx = idx.reshape(1, 2, M, kmax).astype(np.int32)
+    cnt = np.full((1, 2, M), kmax, np.int32)
+    out = block_sparse_attention(*qkv, torch.from_numpy(idx).to(cuda),
+                                 torch.from_numpy(cnt).to(cuda), bs, causal=False)
+    want = O.sparse_attention(*(x.float().cpu().numpy() for x in qkv), idx, cnt, bs, causal=False)
+    assert np.abs(out.float().cpu().numpy() - want).max() <= ATOL["bf16"]
