@@ -51,8 +51,9 @@ struct SumArgs {
 };
 
 // One workgroup of 16 waves per 64 keys: wave w sums the rows (b, h, query)
-// w, w + 16, ..; the waves' sums are added in order. 16-bit weights: the sum is
-// rounded to their type before it is added, as a torch sum of them is.
+// w, w + 16, .., eight at a time, as trees of additions; so are the waves' sums.
+// 16-bit weights: the sum is rounded to their type before it is added, as a
+// torch sum of them is.
 constexpr int SUM_WAVES = 16;
 template <typename T>
 __global__ __launch_bounds__(64 * SUM_WAVES) void key_sums_kernel(SumArgs a) {
@@ -82,15 +83,20 @@ __global__ __launch_bounds__(64 * SUM_WAVES) void key_sums_kernel(SumArgs a) {
             x[u] = f16_to_f32(static_cast<const uint16_t*>(a.a)[off]);
         }
       }
-#pragma unroll
-      for (int u = 0; u < U; ++u) sum += x[u];
+      sum += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
     }
   }
   part[w][lane] = sum;
   __syncthreads();
   if (w != 0 || key >= a.n_out) return;
+  float y[SUM_WAVES];
 #pragma unroll
-  for (int i = 1; i < SUM_WAVES; ++i) sum += part[i][lane];
+  for (int i = 0; i < SUM_WAVES; ++i) y[i] = part[i][lane];
+#pragma unroll
+  for (int n = SUM_WAVES / 2; n >= 1; n >>= 1)
+#pragma unroll
+    for (int i = 0; i < n; ++i) y[i] = y[2 * i] + y[2 * i + 1];
+  sum = y[0];
   if constexpr (std::is_same<T, bf16_t>::value)
     sum = bf16_to_f32(f32_to_bf16(sum));
   else if constexpr (std::is_same<T, f16_t>::value)

@@ -80,6 +80,30 @@ def test_importance_update(cuda, dt, B, H, Nq, Nk, n_old):
     torch.testing.assert_close(got.double(), base, rtol=ulp, atol=1e-7)
 
 
+@gpu
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,Nq,Nk", [(32, 1, 4500), (7, 5, 3000), (32, 16, 4500), (3, 171, 130),
+                                     (32, 128, 12000), (8, 32, 32768)])
+def test_importance_sums_are_as_exact_as_torch(cuda, H, Nq, Nk, dt):
+    """The fp32 sums' rms relative error against float64 is that of a tree of additions: a rounding
+    is uniform within half an ulp, rms 0.4 * 2^-24 of the sum (over mantissas),
+    and a tree's levels add their variances halved each time, 2 in all: 3.4e-8;
+    the eight-row steps of a wave in sequence (32 at most, in each of 16 waves: 2/3
+    more) make it 3.9e-8, and 5.2e-8 is allowed. 16 terms in sequence alone would
+    give sqrt(16 / 3) * 0.4 * 2^-24 = 5.5e-8."""
+    from cab_attention.scoring import ImportanceTracker
+    g = torch.Generator(device=cuda).manual_seed(Nk)
+    w = torch.softmax(torch.randn((1, H, Nq, Nk), generator=g, device=cuda), -1).to(dt)
+    t = ImportanceTracker(device="cuda")
+    t.update(w)
+    want = w.double().sum((0, 1, 2))
+    if dt == torch.float32:
+        rel = (t.get_scores().double() - want) / want
+        assert float(rel.pow(2).mean().sqrt()) <= 5.2e-8
+    else:  # rounded to 8 significant bits: at most 2^-8 of it, plus the fp32 sum's error
+        assert bool(((t.get_scores().double() - want).abs() <= want * (2.0 ** -8 + 1e-6)).all())
+
+
 def test_cache_ops_validation():
     lib = nat.load()
     s = (ctypes.c_int64 * 4)(64, 64, 64, 1)
