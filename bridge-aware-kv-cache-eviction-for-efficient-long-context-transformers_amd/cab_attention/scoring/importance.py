@@ -13,6 +13,23 @@ from ..eviction._select import BRIDGE_NONE, select_positions
 
 _DTYPES = (torch.float32, torch.float16, torch.bfloat16)
 
+def _kernel_sums(rows: int, n_k: int) -> bool:
+    """Whether ``cab_key_sums`` takes a sum over ``rows`` (batch x heads x queries)
+    of ``n_k`` keys; torch's sum the rest. The kernel's workgroups are one per 64
+    keys, each over all rows: one launch instead of several, but too few of them
+    where many rows meet few keys, and slower than torch's wide loads once they
+    run in several rounds. bf16 (fp32), us an update, torch -> kernel:
+    32 rows of 4500 keys 13.3 -> 6.5 (9.2 -> 6.3), 512 of 300 15.8 -> 13.3
+    (12.1 -> 11.7), 512 of 24000 29.6 -> 25.5 (28.4 -> 22.1), 512 of 32768 24.1 ->
+    25.8; 256 of 32768 14.5 -> 13.2 (13.3 -> 12.5), 256 of 50000 20.1 -> 25.1; 8 of
+    131072 13.0 -> 6.8, 64 of 131072 14.2 -> 14.8 (9.8 -> 14.1); 1024 of 8192 16.7 ->
+    25.2 (14.0 -> 22.3), 1024 of 12000 52.2 -> 31.0 (50.0 -> 23.7), 4096 of 24000
+    196 -> 189 (290 -> 155), 16000 of 500 23 -> 424. The fp32 sums' rms error is not
+    above torch's anywhere in it."""
+    if n_k <= 24000:
+        return rows <= 512 or (n_k >= 12000 and rows <= 4096)
+    return rows * n_k <= (1 << 23 if n_k <= 32768 else 1 << 20)
+
 
 class ImportanceTracker:
     """Running sum of the attention each cached position receives."""
@@ -52,6 +69,8 @@ class ImportanceTracker:
                 or (w.requires_grad and torch.is_grad_enabled()) or not nat.addressable(w)):
             return False
         B, H, n_q, n_k = w.shape
+        if not _kernel_sums(B * H * n_q, n_k):
+            return False
         if old is None:
             n_old = 0
         elif (old.device != w.device or old.dtype != torch.float32 or old.dim() != 1
