@@ -19,15 +19,33 @@ def _rows_aligned(t: torch.Tensor) -> bool:
 _APPEND_DTYPES = (torch.bfloat16, torch.float16, torch.float32)
 
 
+def _kernel_appends(k: torch.Tensor, v: torch.Tensor) -> bool:
+    """Whether ``cab_kv_append`` takes the copy; torch the rest. One launch for K
+    and V wins while launches are what counts (6.9 against 9.6 us up to 2^20
+    values). Above, rows off 16-byte boundaries go one value at a time (8 heads x
+    4500 rows x 128 in bf16, us, torch -> kernel: 11.0 -> 18.7 one value off, 13.3 ->
+    18.6 every other value) and torch's copies are faster; aligned rows stay (10.5 ->
+    7.1, transposed 20.0 -> 7.2), contiguous ones to 2^27 bytes (fp32, 40000 rows:
+    115 -> 121)."""
+    if k.numel() <= 1 << 20:
+        return True
+    if not (_rows_aligned(k) and _rows_aligned(v)):
+        return False
+    return k.numel() * k.element_size() <= 1 << 27 or not (k.is_contiguous() and v.is_contiguous())
+
+
 def append_rows(k: torch.Tensor, v: torch.Tensor, k_dst: torch.Tensor, v_dst: torch.Tensor,
                 row: int) -> bool:
     """Copies ``k``, ``v`` ``[B, H, n, D]`` to rows ``row ..`` of the buffers
     ``[B, H, capacity, >= D]`` (one stride set, contiguous last dim) in one
     launch (``cab_kv_append``). False, and nothing done, for what the kernel
-    does not take (another device or dtype, gradients to record, a transform)."""
+    does not take (another device or dtype, gradients to record, a transform) or
+    does more slowly than torch."""
     dev = k_dst.device
     if (dev.type != "cuda" or k.device != dev or v.device != dev
-            or not nat.addressable(k, v, k_dst, v_dst) or k.dtype not in _APPEND_DTYPES or k_dst.dtype != k.dtype
+            or not nat.addressable(k, v, k_dst, v_dst)
+            or k.dtype not in _APPEND_DTYPES or k_dst.dtype != k.dtype
+            or not _kernel_appends(k, v)
             or (torch.is_grad_enabled() and (k.requires_grad or v.requires_grad
                                              or k_dst.requires_grad or v_dst.requires_grad))):
         return False

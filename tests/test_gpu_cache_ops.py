@@ -21,6 +21,7 @@ gpu = pytest.mark.gpu
     (1, 2, 7, 64, "strided"),       # last-dim stride 2
     (1, 2, 9, 64, "offset"),        # rows one element past a 16-byte boundary
     (1, 1, 1, 1, "plain"),
+    (1, 8, 1100, 128, "offset"),    # off 16-byte boundaries and long: torch's copies
 ])
 def test_append_matches_copy(cuda, dt, B, H, n, D, layout):
     from cab_attention.cache.store import LayeredKV

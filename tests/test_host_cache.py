@@ -183,3 +183,19 @@ def test_kernels_leave_transforms_to_torch():
     seen.append(nat.addressable(x.as_subclass(type("Sub", (torch.Tensor,), {}))))
     torch.jit.trace(lambda r: (seen.append(nat.addressable(r)), r + 1)[1], x, check_trace=False)
     assert seen == [False] * 4
+
+
+@pytest.mark.parametrize("n,D,layout,kernel", [
+    (1, 128, "offset", True), (1024, 128, "offset", True),   # launches count
+    (1025, 128, "offset", False), (1025, 128, "strided", False), (1500, 100, "plain", False),
+    (1025, 128, "plain", True), (1025, 128, "transposed", True),
+    (65536, 128, "plain", True), (65537, 128, "plain", False), (65537, 128, "transposed", True),
+])
+def test_appends_taken_by_the_kernel(n, D, layout, kernel):
+    from cab_attention.cache.prune import _kernel_appends
+    H, dt = 8, torch.bfloat16
+    x = {"plain": lambda: torch.empty((1, H, n, D), dtype=dt),
+         "transposed": lambda: torch.empty((1, n, H, D), dtype=dt).transpose(1, 2),
+         "strided": lambda: torch.empty((1, H, n, 2 * D), dtype=dt)[..., ::2],
+         "offset": lambda: torch.empty(H * n * D + 1, dtype=dt)[1:].view(1, H, n, D)}[layout]()
+    assert _kernel_appends(x, x) == kernel
