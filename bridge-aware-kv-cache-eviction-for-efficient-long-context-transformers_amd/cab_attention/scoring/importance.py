@@ -13,7 +13,7 @@ from ..eviction._select import BRIDGE_NONE, select_positions
 
 _DTYPES = (torch.float32, torch.float16, torch.bfloat16)
 
-def _kernel_sums(rows: int, n_k: int) -> bool:
+def _kernel_sums(rows: int, n_k: int, key_stride: int = 1) -> bool:
     """Whether ``cab_key_sums`` takes a sum over ``rows`` (batch x heads x queries)
     of ``n_k`` keys; torch's sum the rest. The kernel's workgroups are one per 64
     keys, each over all rows: one launch instead of several, but too few of them
@@ -25,7 +25,11 @@ def _kernel_sums(rows: int, n_k: int) -> bool:
     131072 13.0 -> 6.8, 64 of 131072 14.2 -> 14.8 (9.8 -> 14.1); 1024 of 8192 16.7 ->
     25.2 (14.0 -> 22.3), 1024 of 12000 52.2 -> 31.0 (50.0 -> 23.7), 4096 of 24000
     196 -> 189 (290 -> 155), 16000 of 500 23 -> 424. The fp32 sums' rms error is not
-    above torch's anywhere in it."""
+    above torch's anywhere in it. Keys apart in memory (a transposed tensor) cost a
+    cache line each: 32 rows of 4500 keys 13.8 -> 6.5 (10.2 -> 6.8), 512 of 300 14.2 ->
+    15.8 (10.2 -> 15.8)."""
+    if key_stride != 1 and rows > 32:
+        return False
     if n_k <= 24000:
         return rows <= 512 or (n_k >= 12000 and rows <= 4096)
     return rows * n_k <= (1 << 23 if n_k <= 32768 else 1 << 20)
@@ -69,7 +73,7 @@ class ImportanceTracker:
                 or (w.requires_grad and torch.is_grad_enabled()) or not nat.addressable(w)):
             return False
         B, H, n_q, n_k = w.shape
-        if not _kernel_sums(B * H * n_q, n_k):
+        if not _kernel_sums(B * H * n_q, n_k, w.stride(3)):
             return False
         if old is None:
             n_old = 0

@@ -199,3 +199,14 @@ def test_appends_taken_by_the_kernel(n, D, layout, kernel):
          "strided": lambda: torch.empty((1, H, n, 2 * D), dtype=dt)[..., ::2],
          "offset": lambda: torch.empty(H * n * D + 1, dtype=dt)[1:].view(1, H, n, D)}[layout]()
     assert _kernel_appends(x, x) == kernel
+
+
+@pytest.mark.parametrize("rows,n_k,stride,kernel", [
+    (512, 1, 1, True), (513, 1, 1, False), (512, 24000, 1, True), (16000, 500, 1, False),
+    (4096, 12000, 1, True), (4096, 11999, 1, False), (4097, 12000, 1, False),
+    (256, 32768, 1, True), (257, 32768, 1, False), (8, 131072, 1, True), (9, 131072, 1, False),
+    (1, 2 ** 31, 1, False), (32, 4500, 3, True), (33, 4500, 3, False),
+])
+def test_sums_taken_by_the_kernel(rows, n_k, stride, kernel):
+    from cab_attention.scoring.importance import _kernel_sums
+    assert _kernel_sums(rows, n_k, stride) == kernel
