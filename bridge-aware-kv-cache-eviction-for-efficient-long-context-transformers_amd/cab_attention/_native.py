@@ -194,11 +194,17 @@ def aligned_rows(t: torch.Tensor) -> torch.Tensor:
     return t if rows_aligned(t) else t.clone()
 
 
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
 def addressable(*tensors: torch.Tensor) -> bool:
-    """Whether a kernel may stand in for torch ops on ``tensors``: plain tensors,
-    with no transform (vmap, forward-mode, tracing) that has to see the ops."""
-    return (all(type(t) is torch.Tensor or type(t) is torch.nn.Parameter for t in tensors)
-            and torch._C._functorch.peek_interpreter_stack() is None
+    """Whether a kernel may stand in for torch ops on ``tensors``: plain tensors
+    whose memory holds their values (no negative bit), with no transform (vmap,
+    forward-mode, tracing) that has to see the ops."""
+    for t in tensors:
+        if type(t) not in _PLAIN or t.is_neg():
+            return False
+    return (torch._C._functorch.peek_interpreter_stack() is None
             and torch.autograd.forward_ad._current_level < 0
             and not torch.compiler.is_compiling() and not torch.jit.is_tracing())
 

@@ -111,6 +111,30 @@ def test_importance_sums_are_as_exact_as_torch(cuda, H, Nq, Nk, dt):
         assert bool(((t.get_scores().double() - want).abs() <= want * (2.0 ** -8 + 1e-6)).all())
 
 
+def _negated(shape, dtype, cuda, g):
+    """A tensor that stands for the negated values of its memory."""
+    z = torch.randn((*shape, 2), generator=g).to(dtype).to(cuda)
+    x = torch._neg_view(z[..., 0].contiguous())
+    assert x.is_neg() and type(x) is torch.Tensor
+    return x
+
+
+@gpu
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_negated_views_keep_their_sign(cuda, dt):
+    from cab_attention.cache.store import LayeredKV
+    from cab_attention.scoring import ImportanceTracker
+    g = torch.Generator().manual_seed(3)
+    k, v, w = (_negated((1, 2, 5, 64), dt, cuda, g) for _ in range(3))
+    store = LayeredKV()
+    store.append(0, k, v)
+    assert torch.equal(store.view(0)[0], k.resolve_neg())
+    assert torch.equal(store.view(0)[1], v.resolve_neg())
+    t = ImportanceTracker(device="cuda")
+    t.update(w)
+    torch.testing.assert_close(t.get_scores(), w.resolve_neg().sum((0, 1, 2)).float())
+
+
 def test_cache_ops_validation():
     lib = nat.load()
     s = (ctypes.c_int64 * 4)(64, 64, 64, 1)

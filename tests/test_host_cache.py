@@ -181,8 +181,9 @@ def test_kernels_leave_transforms_to_torch():
     with torch.autograd.forward_ad.dual_level():
         seen.append(nat.addressable(torch.autograd.forward_ad.make_dual(x, x)))
     seen.append(nat.addressable(x.as_subclass(type("Sub", (torch.Tensor,), {}))))
+    seen.append(nat.addressable(torch._neg_view(x)))
     torch.jit.trace(lambda r: (seen.append(nat.addressable(r)), r + 1)[1], x, check_trace=False)
-    assert seen == [False] * 4
+    assert seen == [False] * 5
 
 
 @pytest.mark.parametrize("n,D,layout,kernel", [
