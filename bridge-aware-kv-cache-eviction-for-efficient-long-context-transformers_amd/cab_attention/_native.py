@@ -14,6 +14,7 @@ import pathlib
 import threading
 
 import torch
+from torch.utils._device import DeviceContext
 
 # The in-tree build; CAB_HIP_LIB names another build of the same library (the
 # host-sanitized one that tests/test_host_sanitizers.py runs the ABI checks on).
@@ -200,13 +201,22 @@ _PLAIN = (torch.Tensor, torch.nn.Parameter)
 def addressable(*tensors: torch.Tensor) -> bool:
     """Whether a kernel may stand in for torch ops on ``tensors``: plain tensors
     whose memory holds their values (no negative bit), with no transform (vmap,
-    forward-mode, tracing) that has to see the ops."""
+    forward-mode, tracing) and no mode that has to see the ops."""
     for t in tensors:
         if type(t) not in _PLAIN or t.is_neg():
             return False
     return (torch._C._functorch.peek_interpreter_stack() is None
             and torch.autograd.forward_ad._current_level < 0
-            and not torch.compiler.is_compiling() and not torch.jit.is_tracing())
+            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+            and torch._C._len_torch_dispatch_stack() == 0
+            and (torch._C._len_torch_function_stack() == 0 or _only_device_modes()))
+
+
+def _only_device_modes() -> bool:
+    """Whether the active function modes are default devices alone, which no op on
+    existing tensors asks."""
+    return all(type(m) is DeviceContext
+               for m in torch.overrides._get_current_function_mode_stack())
 
 
 _SAME_DEVICE = contextlib.nullcontext()

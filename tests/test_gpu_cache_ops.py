@@ -135,6 +135,25 @@ def test_negated_views_keep_their_sign(cuda, dt):
     torch.testing.assert_close(t.get_scores(), w.resolve_neg().sum((0, 1, 2)).float())
 
 
+@gpu
+def test_dispatch_modes_see_the_ops(cuda):
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from cab_attention.cache.store import LayeredKV
+    from cab_attention.scoring import ImportanceTracker
+
+    class Names(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            names.append(func.overloadpacket.__name__)
+            return func(*args, **(kwargs or {}))
+
+    names = []
+    k, w = torch.rand((1, 2, 3, 64), device=cuda), torch.rand((1, 2, 3, 7), device=cuda)
+    with Names():
+        LayeredKV().append(0, k, k)
+        ImportanceTracker(device="cuda").update(w)
+    assert names.count("copy_") == 2 and "sum" in names
+
+
 def test_cache_ops_validation():
     lib = nat.load()
     s = (ctypes.c_int64 * 4)(64, 64, 64, 1)

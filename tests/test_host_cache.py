@@ -186,6 +186,34 @@ def test_kernels_leave_transforms_to_torch():
     assert seen == [False] * 5
 
 
+def test_kernels_leave_modes_to_torch():
+    """Dispatch and function modes (make_fx's tracing, op counters) see the ops; a
+    default device has no say in ops on existing tensors."""
+    from cab_attention import _native as nat
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    x = torch.zeros(2, 3)
+    seen = []
+    make_fx(lambda r: (seen.append(nat.addressable(x)), r + 1)[1])(x)
+    for mode in (Function(), Dispatch()):
+        with mode:
+            seen.append(nat.addressable(x))
+    assert seen == [False] * 3
+    with torch.device("cpu"):
+        assert nat.addressable(x)
+    assert nat.addressable(x)
+
+
 @pytest.mark.parametrize("n,D,layout,kernel", [
     (1, 128, "offset", True), (1024, 128, "offset", True),   # launches count
     (1025, 128, "offset", False), (1025, 128, "strided", False), (1500, 100, "plain", False),
