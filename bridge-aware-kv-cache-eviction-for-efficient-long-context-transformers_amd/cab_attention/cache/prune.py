@@ -56,6 +56,7 @@ def append_rows(k: torch.Tensor, v: torch.Tensor, k_dst: torch.Tensor, v_dst: to
                                       nat.strides4(k), nat.strides4(v), nat.strides4(k_dst), row,
                                       nat.stream_ptr(dev))
     nat.check("cab_kv_append", st)
+    nat.wrote(k_dst, v_dst)
     return True
 
 

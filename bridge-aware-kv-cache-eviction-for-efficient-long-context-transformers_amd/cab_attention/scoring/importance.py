@@ -89,6 +89,8 @@ class ImportanceTracker:
                                          nat.strides4(w), nat.ptr(old), n_old, sums.data_ptr(),
                                          nat.stream_ptr(w.device))
         nat.check("cab_key_sums", st)
+        if sums is old:
+            nat.wrote(sums)
         self.cumulative_scores = sums
         self.total_queries += n_q
         return True

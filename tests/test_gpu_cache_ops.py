@@ -154,6 +154,30 @@ def test_dispatch_modes_see_the_ops(cuda):
     assert names.count("copy_") == 2 and "sum" in names
 
 
+@gpu
+def test_in_place_writes_are_seen_by_autograd(cuda):
+    """What a backward pass has saved and an update then writes over raises, as for
+    torch's own in-place ops."""
+    from cab_attention.cache.store import LayeredKV
+    from cab_attention.scoring import ImportanceTracker
+    t = ImportanceTracker(device="cuda")
+    w = torch.rand((1, 2, 3, 7), device=cuda)
+    t.update(w)
+    x = torch.ones(7, device=cuda, requires_grad=True)
+    y = (x * t.get_scores()).sum()
+    before = t.get_scores()._version
+    t.update(w)
+    assert t.get_scores()._version > before
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.backward()
+    store, k = LayeredKV(), torch.rand((1, 2, 3, 64), device=cuda)
+    store.append(0, k, k)
+    kept = store.view(0)
+    before = [s._version for s in kept]
+    store.append(0, k, k)
+    assert all(s._version > b for s, b in zip(kept, before))
+
+
 def test_cache_ops_validation():
     lib = nat.load()
     s = (ctypes.c_int64 * 4)(64, 64, 64, 1)
