@@ -219,6 +219,12 @@ def _only_device_modes() -> bool:
                for m in torch.overrides._get_current_function_mode_stack())
 
 
+def closed(t: torch.Tensor) -> bool:
+    """Whether torch refuses in-place writes into ``t`` here (an inference tensor
+    outside inference mode)."""
+    return t.is_inference() and not torch.is_inference_mode_enabled()
+
+
 def wrote(*tensors: torch.Tensor) -> None:
     """Tells autograd of a kernel's writes into ``tensors``, as torch's in-place ops
     do: a backward pass that saved them raises instead of reading new values."""

@@ -45,7 +45,7 @@ def append_rows(k: torch.Tensor, v: torch.Tensor, k_dst: torch.Tensor, v_dst: to
     if (dev.type != "cuda" or k.device != dev or v.device != dev
             or not nat.addressable(k, v, k_dst, v_dst)
             or k.dtype not in _APPEND_DTYPES or k_dst.dtype != k.dtype
-            or not _kernel_appends(k, v)
+            or not _kernel_appends(k, v) or nat.closed(k_dst)
             or (torch.is_grad_enabled() and (k.requires_grad or v.requires_grad
                                              or k_dst.requires_grad or v_dst.requires_grad))):
         return False

@@ -82,6 +82,8 @@ class ImportanceTracker:
             return False
         else:
             n_old = old.numel()
+            if n_old >= n_k and nat.closed(old):
+                return False
         # Totals that reach far enough are added to in place, shorter ones extended.
         sums = old if n_old >= n_k else torch.empty(n_k, dtype=torch.float32, device=w.device)
         with nat.on_device(w.device):

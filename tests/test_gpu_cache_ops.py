@@ -178,6 +178,24 @@ def test_in_place_writes_are_seen_by_autograd(cuda):
     assert all(s._version > b for s, b in zip(kept, before))
 
 
+@gpu
+def test_inference_tensors_stay_closed_outside_inference_mode(cuda):
+    from cab_attention.cache.store import LayeredKV
+    from cab_attention.scoring import ImportanceTracker
+    t, store = ImportanceTracker(device="cuda"), LayeredKV()
+    w, k = torch.rand((1, 2, 3, 7), device=cuda), torch.rand((1, 2, 3, 64), device=cuda)
+    with torch.inference_mode():
+        for _ in range(2):
+            t.update(w)
+            store.append(0, k, k)
+    torch.testing.assert_close(t.get_scores(), 2 * w.sum((0, 1, 2)))
+    assert store.length(0) == 6
+    with pytest.raises(RuntimeError, match="[Ii]nference"):
+        t.update(w)
+    with pytest.raises(RuntimeError, match="[Ii]nference"):
+        store.append(0, k, k)
+
+
 def test_cache_ops_validation():
     lib = nat.load()
     s = (ctypes.c_int64 * 4)(64, 64, 64, 1)
