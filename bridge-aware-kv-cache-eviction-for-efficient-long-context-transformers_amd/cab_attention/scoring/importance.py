@@ -72,6 +72,8 @@ class ImportanceTracker:
         if (w.device.type != "cuda" or w.dim() != 4 or w.dtype not in _DTYPES or w.numel() == 0
                 or (w.requires_grad and torch.is_grad_enabled()) or not nat.addressable(w)):
             return False
+        if w.dtype != torch.float32 and torch.is_autocast_enabled("cuda"):
+            return False  # autocast sums in fp32 and does not round
         B, H, n_q, n_k = w.shape
         if not _kernel_sums(B * H * n_q, n_k, w.stride(3)):
             return False

@@ -196,6 +196,20 @@ def test_inference_tensors_stay_closed_outside_inference_mode(cuda):
         store.append(0, k, k)
 
 
+@gpu
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_importance_update_under_autocast(cuda, dt):
+    """Autocast sums in fp32: 16-bit weights' sums are not rounded to their type."""
+    from cab_attention.scoring import ImportanceTracker
+    g = torch.Generator(device=cuda).manual_seed(4)
+    w = torch.softmax(torch.randn((1, 8, 16, 300), generator=g, device=cuda), -1).to(dt)
+    t = ImportanceTracker(device="cuda")
+    with torch.autocast("cuda", dtype=dt):
+        t.update(w)
+    want = w.double().sum((0, 1, 2))
+    torch.testing.assert_close(t.get_scores().double(), want, rtol=1e-6, atol=0.0)
+
+
 def test_cache_ops_validation():
     lib = nat.load()
     s = (ctypes.c_int64 * 4)(64, 64, 64, 1)
