@@ -174,7 +174,13 @@ def flash_attention_with_cumulative_scores(
         old = old.float().contiguous()
     scores = old
     if old.shape[2] < N_k:
-        scores = torch.empty((B, H, N_k), dtype=torch.float32, device=q.device)
+        if (old.requires_grad and torch.is_grad_enabled()) or not nat.addressable(old):
+            # Extended by torch, so that the longer totals stay in the graph (or
+            # transform) the old ones come from.
+            extension = torch.zeros(B, H, N_k - old.shape[2], dtype=torch.float32, device=q.device)
+            scores = old = torch.cat([old, extension], dim=2)
+        else:
+            scores = torch.empty((B, H, N_k), dtype=torch.float32, device=q.device)
     return _dense(q, k, v, scale, causal, old=old, scores=scores)[0], scores
 
 

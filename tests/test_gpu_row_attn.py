@@ -95,6 +95,23 @@ def test_masked_values_and_far_maxima(cuda):
     np.testing.assert_allclose(np64(lse), w_lse, atol=LSE_ATOL["bf16"], rtol=1e-4)
 
 
+def test_shorter_totals_carry_their_gradient(cuda):
+    """Totals that are extended to new keys stay in the graph they come from (the
+    call's own totals have none)."""
+    from cab_attention.kernels import flash_attention_with_cumulative_scores
+    q, k, v = (seeded((1, 2, n, 64), n, torch.bfloat16).to(cuda) for n in (3, 40, 40))
+    old = torch.rand((1, 2, 33), device=cuda, requires_grad=True)
+    _, sc = flash_attention_with_cumulative_scores(q, k, v, old * 2.0)
+    _, plain = flash_attention_with_cumulative_scores(q, k, v, (old * 2.0).detach())
+    assert torch.equal(sc.detach(), plain)
+    sc.square().sum().backward()
+    torch.testing.assert_close(old.grad, 4.0 * plain[..., :33])
+    neg = torch._neg_view(old.detach())
+    _, sc = flash_attention_with_cumulative_scores(q, k, v, neg)
+    _, plain = flash_attention_with_cumulative_scores(q, k, v, -old.detach())
+    assert torch.equal(sc, plain)
+
+
 @pytest.mark.parametrize("dt", ["bf16", "fp32"])
 def test_flash_fwd_workspace_decides_the_path(cuda, dt):
     """cab_flash_attn_fwd takes its documented workspace whatever path runs: for
