@@ -168,11 +168,11 @@ def require_device(*tensors: torch.Tensor) -> torch.device:
     return dev
 
 
-_I64x4 = ctypes.c_int64 * 4
+I64x4 = ctypes.c_int64 * 4
 
 
 def strides4(t: torch.Tensor):
-    return _I64x4(*t.stride())
+    return I64x4(*t.stride())
 
 
 def rows_aligned(t: torch.Tensor) -> bool:
@@ -196,20 +196,26 @@ def aligned_rows(t: torch.Tensor) -> torch.Tensor:
 
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
+# Looked up once: a decode step asks addressable() per layer.
+_is_compiling = torch.compiler.is_compiling
+_is_tracing = torch._C._is_tracing
+_interpreter = torch._C._functorch.peek_interpreter_stack
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+_function_modes = torch._C._len_torch_function_stack
+_forward_ad = torch.autograd.forward_ad
 
 
 def addressable(*tensors: torch.Tensor) -> bool:
     """Whether a kernel may stand in for torch ops on ``tensors``: plain tensors
     whose memory holds their values (no negative bit), with no transform (vmap,
     forward-mode, tracing) and no mode that has to see the ops."""
+    if _is_compiling():
+        return False
     for t in tensors:
         if type(t) not in _PLAIN or t.is_neg():
             return False
-    return (torch._C._functorch.peek_interpreter_stack() is None
-            and torch.autograd.forward_ad._current_level < 0
-            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
-            and torch._C._len_torch_dispatch_stack() == 0
-            and (torch._C._len_torch_function_stack() == 0 or _only_device_modes()))
+    return (_interpreter() is None and _forward_ad._current_level < 0 and not _is_tracing()
+            and not _dispatch_modes() and (not _function_modes() or _only_device_modes()))
 
 
 def _only_device_modes() -> bool:
@@ -242,9 +248,12 @@ def on_device(device: torch.device):
     return torch.cuda.device(device)
 
 
+raw_stream = torch._C._cuda_getCurrentRawStream  # of a device index
+
+
 def stream_ptr(device: torch.device) -> int:
     index = torch.cuda.current_device() if device.index is None else device.index
-    return torch._C._cuda_getCurrentRawStream(index)
+    return raw_stream(index)
 
 
 def ptr(t):

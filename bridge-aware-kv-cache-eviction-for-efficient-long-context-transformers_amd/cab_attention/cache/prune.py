@@ -16,7 +16,8 @@ def _rows_aligned(t: torch.Tensor) -> bool:
     return nat.rows_aligned(t) and (t.shape[3] * t.element_size()) % 16 == 0
 
 
-_APPEND_DTYPES = (torch.bfloat16, torch.float16, torch.float32)
+_APPEND_BYTES = {torch.bfloat16: 2, torch.float16: 2, torch.float32: 4}
+_SMALL = 1 << 20  # values
 
 
 def _kernel_appends(k: torch.Tensor, v: torch.Tensor) -> bool:
@@ -27,7 +28,7 @@ def _kernel_appends(k: torch.Tensor, v: torch.Tensor) -> bool:
     18.6 every other value) and torch's copies are faster; aligned rows stay (10.5 ->
     7.1, transposed 20.0 -> 7.2), contiguous ones to 2^27 bytes (fp32, 40000 rows:
     115 -> 121)."""
-    if k.numel() <= 1 << 20:
+    if k.numel() <= _SMALL:
         return True
     if not (_rows_aligned(k) and _rows_aligned(v)):
         return False
@@ -41,20 +42,25 @@ def append_rows(k: torch.Tensor, v: torch.Tensor, k_dst: torch.Tensor, v_dst: to
     launch (``cab_kv_append``). False, and nothing done, for what the kernel
     does not take (another device or dtype, gradients to record, a transform) or
     does more slowly than torch."""
-    dev = k_dst.device
-    if (dev.type != "cuda" or k.device != dev or v.device != dev
-            or not nat.addressable(k, v, k_dst, v_dst)
-            or k.dtype not in _APPEND_DTYPES or k_dst.dtype != k.dtype
-            or not _kernel_appends(k, v) or nat.closed(k_dst)
+    es = _APPEND_BYTES.get(k.dtype)
+    index = k_dst.get_device()
+    if (es is None or k_dst.dtype != k.dtype or not k_dst.is_cuda or k.get_device() != index
+            or v.get_device() != index or not nat.addressable(k, v)
+            or type(k_dst) is not torch.Tensor or type(v_dst) is not torch.Tensor
+            or nat.closed(k_dst)
             or (torch.is_grad_enabled() and (k.requires_grad or v.requires_grad
                                              or k_dst.requires_grad or v_dst.requires_grad))):
         return False
     B, H, n, D = k.shape
-    with nat.on_device(dev):
+    if B * H * n * D > _SMALL and not _kernel_appends(k, v):
+        return False
+    k_st, v_st = k.stride(), v.stride()
+    k_arr = nat.I64x4(*k_st)
+    with nat.on_device(k_dst.device):
         st = nat.load().cab_kv_append(k.data_ptr(), v.data_ptr(), k_dst.data_ptr(),
-                                      v_dst.data_ptr(), k.element_size(), B, H, n, D,
-                                      nat.strides4(k), nat.strides4(v), nat.strides4(k_dst), row,
-                                      nat.stream_ptr(dev))
+                                      v_dst.data_ptr(), es, B, H, n, D, k_arr,
+                                      k_arr if v_st == k_st else nat.I64x4(*v_st),
+                                      nat.strides4(k_dst), row, nat.raw_stream(index))
     nat.check("cab_kv_append", st)
     nat.wrote(k_dst, v_dst)
     return True

@@ -184,6 +184,9 @@ def test_kernels_leave_transforms_to_torch():
     seen.append(nat.addressable(torch._neg_view(x)))
     torch.jit.trace(lambda r: (seen.append(nat.addressable(r)), r + 1)[1], x, check_trace=False)
     assert seen == [False] * 5
+    compiled = torch.compile(lambda r: r + 1 if nat.addressable(r) else r - 1, backend="eager",
+                             fullgraph=True)
+    assert torch.equal(compiled(x), x - 1)
 
 
 def test_kernels_leave_modes_to_torch():
