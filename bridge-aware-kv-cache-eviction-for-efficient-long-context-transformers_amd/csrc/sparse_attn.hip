@@ -706,9 +706,11 @@ __global__ __launch_bounds__(256, DT == CAB_F32 ? 1 : 2) void attn_fwd_kernel(At
   const int64_t kblk_bytes = BS * krow_bytes;
   // Bytes of block j's valid rows: to the end of the last one, which lies past
   // rows * krow_bytes where rows overlap (a token stride below D).
-  const uint32_t kfull = static_cast<uint32_t>((BS - 1) * krow_bytes + 2 * HD);
-  const uint32_t klast = static_cast<uint32_t>((Nk - 1) % BS * krow_bytes + 2 * HD);
-  auto k_bytes = [&](int j) { return j + 1 < Mk ? kfull : klast; };
+  const uint32_t kpad = krow_bytes < 2 * HD ? static_cast<uint32_t>(2 * HD - krow_bytes) : 0u;
+  auto k_bytes = [&](int j) {
+    const int rows = Nk - j * BS < BS ? Nk - j * BS : BS;
+    return static_cast<uint32_t>(rows * krow_bytes) + kpad;
+  };
   uint32_t koff[NI];
 #pragma unroll
   for (int r = 0; r < NI; ++r) koff[r] = k_lane_off<HD>(NI * w + r, ge.lane, krow_bytes);
@@ -1123,12 +1125,6 @@ __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
   const int64_t krow_bytes = a.ks[2] * 2;
   const int64_t kblk_bytes = BS * krow_bytes;
   const int64_t vrow_bytes = VROW ? a.vs[2] * 2 : 0;
-  // Descriptor sizes of a whole block and of the last one (see attn_fwd_kernel).
-  const int last_row = (Nk - 1) % BS;
-  const uint32_t kfull = static_cast<uint32_t>((BS - 1) * krow_bytes + 2 * HD);
-  const uint32_t klast = static_cast<uint32_t>(last_row * krow_bytes + 2 * HD);
-  const uint32_t vfull = static_cast<uint32_t>((BS - 1) * vrow_bytes + 2 * HD);
-  const uint32_t vlast = static_cast<uint32_t>(last_row * vrow_bytes + 2 * HD);
   // Lane offset of load r: row = ROWS_PER_LOAD (NI w + r) + lane / CPR, whose
   // swizzle is 4 r | lane / 16, so the chunk's byte is loff ^ 64 r.
   const uint32_t lrow = G::ROWS_PER_LOAD * NI * w + lane / G::CPR;
@@ -1145,10 +1141,11 @@ __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
     static_assert(NDS % 2 == 0 && NDT % (NDS / 2) == 0, "staging parts split over S and P V");
     char* kl = reinterpret_cast<char*>(kst) + w * NI * 1024;
     char* vl = reinterpret_cast<char*>(vst) + w * NI * 1024;
-    const bool whole = j + 1 < Mk;
-    const sgpr_rsrc_t krs = make_sgpr_rsrc(kbytes + j * kblk_bytes, whole ? kfull : klast);
+    const int rows = Nk - j * BS < BS ? Nk - j * BS : BS;
+    const sgpr_rsrc_t krs =
+        make_sgpr_rsrc(kbytes + j * kblk_bytes, static_cast<uint32_t>(rows * krow_bytes));
     const sgpr_rsrc_t vrs =
-        VROW ? make_sgpr_rsrc(vtbytes + j * BS * vrow_bytes, whole ? vfull : vlast)
+        VROW ? make_sgpr_rsrc(vtbytes + j * BS * vrow_bytes, static_cast<uint32_t>(rows * vrow_bytes))
              : make_sgpr_rsrc(vtbytes + static_cast<int64_t>(j) * TILE_BYTES, TILE_BYTES);
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
@@ -1583,7 +1580,7 @@ constexpr int ks_q_bytes() { return (F32 ? 64 : 32) * HD; }
 template <int HD, bool F32>
 constexpr int ks_stage_bytes() { return ks_q_bytes<HD, F32>() + 4 * 256; }
 
-template <cab_dtype_t DT, int NW, int HD>
+template <cab_dtype_t DT, int NW, int HD, bool QPAD>
 __global__ __launch_bounds__(64 * NW) void key_score_kernel(KeyScoreArgs a) {
   constexpr int NDS = Dims<HD>::NDS;
   constexpr bool F32 = DT == CAB_F32;
@@ -1660,8 +1657,9 @@ __global__ __launch_bounds__(64 * NW) void key_score_kernel(KeyScoreArgs a) {
     const int q0 = 16 * tile_of(it);
     const uint32_t rows = static_cast<uint32_t>(min(16, a.Nq - q0));
     if (qstager) {
-      const brsrc_t qrs =
-          make_rsrc(qb + static_cast<int64_t>(q0) * a.qs[2] * ESZ, (rows - 1) * qrow + HD * ESZ);
+      // (QPAD: rows that overlap end past rows * qrow)
+      const brsrc_t qrs = make_rsrc(qb + static_cast<int64_t>(q0) * a.qs[2] * ESZ,
+                                    QPAD ? (rows - 1) * qrow + HD * ESZ : rows * qrow);
       if constexpr (F32) {
         bdma16(qrs, q_voff, 0, st + 2048 * w);
         bdma16(qrs, q_voff + 16u, 0, st + 2048 * w + 1024);
@@ -1938,9 +1936,12 @@ struct AttnGeom {
   int list;
 };
 
-// Whether attn_pair_kernel takes a call.
-bool pair_path(cab_dtype_t dtype, const AttnGeom& g, int32_t kmax, bool sub) {
-  return dtype != CAB_F32 && !sub && pair_enabled() &&
+// Whether attn_pair_kernel takes a call. (Its descriptors are sized rows * stride,
+// which cuts rows that overlap: those of K go to attn_fwd_kernel. Sized to the
+// last row's end, the pair kernel ran 0.3 to 0.8 % longer.)
+bool pair_path(cab_dtype_t dtype, const AttnGeom& g, int32_t kmax, bool sub,
+               const int64_t* k_strides) {
+  return dtype != CAB_F32 && !sub && pair_enabled() && k_strides[2] >= g.D &&
          ((g.list == LIST_LDS && kmax <= PAIR_KMAX) || g.list == LIST_DENSE);
 }
 // ... and reads V's rows instead of tiles packed ahead of it: where a key block
@@ -2003,7 +2004,7 @@ cab_status_t launch_attn(const char* fn, const void* q, const void* k, const voi
   a.splits = splits;
   a.po = parts;
   a.pml = parts ? parts + static_cast<int64_t>(splits) * a.BH * a.N * g.D : nullptr;
-  if (pair_path(dtype, g, kmax, submask != nullptr)) {
+  if (pair_path(dtype, g, kmax, submask != nullptr, k_strides)) {
     const dim3 pgrid(static_cast<unsigned>(g.B * g.H * ((M + 1) / 2)));
     auto go = [&](auto dt_tag, auto hd_tag) {
       constexpr cab_dtype_t DT = decltype(dt_tag)::value;
@@ -2211,7 +2212,7 @@ extern "C" cab_status_t cab_block_sparse_attn_fwd(
   }
   const int32_t k64 = block_size == BS ? kmax : static_cast<int32_t>(tl.K64);
   const bool vrows = v_rows(v_strides, D, k64) &&
-                     pair_path(dtype, sparse_geom(B, H, N, D, k64), k64, block_size < BS);
+                     pair_path(dtype, sparse_geom(B, H, N, D, k64), k64, block_size < BS, k_strides);
   if (dtype == CAB_F32)
     st = launch_pack_split("cab_block_sparse_attn_fwd/pack_split", k, k_strides, v, v_strides, B,
                            H, N, D, workspace, s);
@@ -2308,18 +2309,27 @@ cab_status_t launch_key_scores(const char* fn, const void* q, const void* k, con
   a.causal = causal ? 1 : 0;
   a.scale_log2 = static_cast<float>(static_cast<double>(scale) * 1.4426950408889634);
   const dim3 grid(static_cast<unsigned>(B * H * a.Mkg));
-  auto launch = [&](auto hd_tag) {
-    constexpr int HDT = decltype(hd_tag)::value;
+  auto launch = [&](auto hd_tag, auto pad_tag) {
+    constexpr int HD = decltype(hd_tag)::value;
+    constexpr bool QPAD = decltype(pad_tag)::value;
+    const dim3 block(64 * KS_WAVES);
     switch (dtype) {
-      case CAB_BF16: key_score_kernel<CAB_BF16, KS_WAVES, HDT><<<grid, 64 * KS_WAVES, 0, s>>>(a); break;
-      case CAB_F16: key_score_kernel<CAB_F16, KS_WAVES, HDT><<<grid, 64 * KS_WAVES, 0, s>>>(a); break;
-      default: key_score_kernel<CAB_F32, KS_WAVES, HDT><<<grid, 64 * KS_WAVES, 0, s>>>(a); break;
+      case CAB_BF16: key_score_kernel<CAB_BF16, KS_WAVES, HD, QPAD><<<grid, block, 0, s>>>(a); break;
+      case CAB_F16: key_score_kernel<CAB_F16, KS_WAVES, HD, QPAD><<<grid, block, 0, s>>>(a); break;
+      default: key_score_kernel<CAB_F32, KS_WAVES, HD, QPAD><<<grid, block, 0, s>>>(a); break;
     }
   };
-  if (D == 64)
-    launch(std::integral_constant<int, 64>{});
+  auto with_hd = [&](auto pad_tag) {
+    if (D == 64)
+      launch(std::integral_constant<int, 64>{}, pad_tag);
+    else
+      launch(std::integral_constant<int, 128>{}, pad_tag);
+  };
+  // Queries that overlap (a token stride below D) take the padded descriptors.
+  if (q_strides[2] < D)
+    with_hd(std::true_type{});
   else
-    launch(std::integral_constant<int, 128>{});
+    with_hd(std::false_type{});
   return launch_status(fn);
 }
 
@@ -2443,7 +2453,7 @@ cab_status_t dense_forward(const char* fn, const void* q, const void* k, const v
     lse = reinterpret_cast<float*>(static_cast<char*>(workspace) + plan.off_lse);
   if (scores && (st = check_score_rows(fn, q, lse, q_strides, esize)) != CAB_OK) return st;
   const AttnGeom g{B, H, H_kv, N_q, N_k, D, N_k - N_q, LIST_DENSE};
-  const bool vrows = v_rows(v_strides, D, dense_visits(g, causal)) && pair_path(dtype, g, 1, false);
+  const bool vrows = v_rows(v_strides, D, dense_visits(g, causal)) && pair_path(dtype, g, 1, false, k_strides);
   if (dtype == CAB_F32)
     st = launch_pack_split(fn, k, k_strides, v, v_strides, B, H_kv, N_k, D, workspace, s);
   else if (!vrows)
