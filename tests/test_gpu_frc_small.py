@@ -70,3 +70,31 @@ def test_fused_form_has_one_set_of_roundings(cuda, M, dt):
     want = torch.matmul(x, xt)
     bound = M * 2.0 ** -23 * torch.matmul(x.abs(), xt.abs()) + 1e-9  # fp32 sums of exact products
     assert bool(((frc.cpu().double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("M,D", [(2, 64), (5, 128), (31, 72), (32, 128), (33, 256), (64, 64), (100, 128),
+                                 (127, 24), (128, 128)])
+@pytest.mark.parametrize("dt", ["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("formula", ["additive", "multiplicative"])
+@pytest.mark.parametrize("diagnostics", [True, False])
+def test_same_bits_as_the_general_kernels(cuda, M, D, dt, formula, diagnostics):
+    """The same matrix once alone (one kernel) and once inside one of 160 blocks (the
+    general kernels) whose added keys score the minimum with every query: their
+    column of Ahat is exactly 0, so they add exact zeros to every sum over keys and
+    leave minimum and maximum as they are."""
+    from cab_attention.kernels import compute_block_frc
+    g = torch.Generator().manual_seed(M * 7 + D)
+    big = 160
+    q, k = (torch.randn((1, 2, big, D), generator=g) for _ in range(2))
+    q[..., -1], k[..., -1] = 1.0, 0.0
+    k[:, :, M - 1:] = 0.0          # key M - 1 is the first that scores the minimum,
+    k[:, :, M - 1:, -1] = -512.0   # -512 * alpha, exact in every type
+    q[:, :, M:] = q[:, :, :1]
+    q, k = (x.to(DTYPES[dt]).to(cuda) for x in (q, k))
+    kw = dict(lambda_redundancy=0.7, formula=formula, diagnostics=diagnostics)
+    small = compute_block_frc(q[:, :, :M].contiguous(), k[:, :, :M].contiguous(), **kw)
+    general = compute_block_frc(q, k, **kw)
+    for a, b in zip(small, general):
+        assert (a is None) == (b is None)
+        if a is not None:
+            assert torch.equal(a, b[:, :, :M, :M])

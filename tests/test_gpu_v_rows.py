@@ -80,8 +80,6 @@ def test_v_rows_far_apart(cuda):
     far = torch.empty((Nk - 1) * step + D, dtype=torch.bfloat16, device=cuda)
     far = far.as_strided((1, 1, Nk, D), (step * Nk, step * Nk, step, 1))
     far.copy_(v)
-    assert torch.equal(flash_attention(q, k, far, causal=True),
-                       flash_attention(q, k, far, causal=True))
     want, _, _ = O.dense_attention_scores(*(x.astype(np.float64) for x in f), causal=True)
     assert np.abs(flash_attention(q, k, far, causal=True).float().cpu().numpy() - want).max() <= ATOL["bf16"]
 
