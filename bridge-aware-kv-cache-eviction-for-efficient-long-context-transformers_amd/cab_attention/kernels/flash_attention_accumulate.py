@@ -71,7 +71,12 @@ def _dense(q, k, v, scale, causal, out=None, want_lse=False, old=None, scores=No
     _check_dense(q, k, v)
     B, H, N_q, D = q.shape
     H_kv, N_k = k.shape[1], k.shape[2]
-    dev = nat.require_device(q, k, v, *(t for t in (old, scores) if t is not None))
+    if scores is None:
+        dev = nat.require_device(q, k, v)
+    elif old is None:
+        dev = nat.require_device(q, k, v, scores)
+    else:
+        dev = nat.require_device(q, k, v, scores, old)
     lib = nat.load()
     dt = nat.dtype_code(q)
     q = nat.aligned_rows(q)
@@ -82,18 +87,20 @@ def _dense(q, k, v, scale, causal, out=None, want_lse=False, old=None, scores=No
     lse = torch.empty((B, H, N_q), dtype=torch.float32, device=dev) if want_lse else None
     if scale is None:
         scale = 1.0 / math.sqrt(D)
-    ks, vs = nat.strides4(k), nat.strides4(v)
+    ks = nat.strides4(k)
+    vs = ks if v.stride() == k.stride() else nat.strides4(v)
+    qs = nat.strides4(q)
     wbytes = lib.cab_flash_attn_scores_workspace_bytes(dt, B, H, H_kv, N_q, N_k, D, ks, vs,
                                                        int(scores is not None))
     ws = torch.empty(max(int(wbytes), 16), dtype=torch.uint8, device=dev)
     with nat.on_device(dev):
         st = lib.cab_flash_attn_scores_fwd(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), dt, B, H, H_kv, N_q, N_k, D,
-            nat.strides4(q), ks, vs, nat.strides4(out), float(scale), int(bool(causal)),
-            out.data_ptr(), nat.ptr(lse), nat.ptr(old), None if old is None else nat.strides4(old),
-            0 if old is None else old.shape[2], nat.ptr(scores),
-            None if scores is None else nat.strides4(scores), ws.data_ptr(), ws.numel(),
-            nat.stream_ptr(dev))
+            qs, ks, vs, qs if out.stride() == q.stride() else nat.strides4(out), float(scale),
+            int(bool(causal)), out.data_ptr(), nat.ptr(lse), nat.ptr(old),
+            None if old is None else nat.strides4(old), 0 if old is None else old.shape[2],
+            nat.ptr(scores), None if scores is None else nat.strides4(scores), ws.data_ptr(),
+            ws.numel(), nat.stream_ptr(dev))
     nat.check("cab_flash_attn_scores_fwd", st)
     return out, lse
 
