@@ -980,7 +980,6 @@ __device__ __forceinline__ void pair_softmax(PairAcc<HD>& s, int r, f32x4 (&sc)[
 
 // VROW: V is staged as its rows, in K's LDS layout, and the V^T operands come
 // from transposing LDS reads; otherwise from packed V^T tiles (cab_..._packed).
-// ---------------------------------------------------------------------------
 template <cab_dtype_t DT, int LIST, int HD, bool VROW>
 __global__ __launch_bounds__(256, 2) void attn_pair_kernel(AttnArgs a) {
   static_assert(DT != CAB_F32, "16-bit inputs only");

@@ -260,7 +260,10 @@ cab_status_t cab_block_sparse_attn_fwd_packed(const void* q, const void* k, cons
  * q, out: [B,H,N_q,D]; k, v: [B,H_kv,N_k,D] (strides); lse: contiguous fp32
  * [B,H,N_q]. D == 64 or 128; bf16, fp16 or fp32 (fp32: split bf16 MFMA as in
  * cab_block_sparse_attn_fwd). workspace: cab_flash_attn_workspace_bytes()
- * bytes, 16-byte aligned, overwritten.
+ * bytes, 16-byte aligned, overwritten. Token strides below D (overlapping rows,
+ * or 0: one row for all) are taken, here and in the block-sparse calls. A key
+ * a query does not see has weight 0 there, but its V row may enter the same
+ * products: V has to be finite over the call's keys (0 * inf is NaN).
  *
  * cab_attn_key_scores: score[b,h,s] (+)= sum over queries t of
  * exp(q_t . k_s * scale - lse[b,h,t]), i.e. the total softmax probability
